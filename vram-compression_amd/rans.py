@@ -17,6 +17,7 @@ import copy
 import ctypes
 import os
 import subprocess
+import tempfile
 
 import numpy as np
 import torch
@@ -25,9 +26,9 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "librans_hip.so")
-SOURCES = [os.path.join(CSRC, "rans_gemv.hip"), os.path.join(CSRC, "ref32_gemv.hip"),
-           os.path.join(CSRC, "w64_host.cpp")]
-HEADERS = [os.path.join(INCLUDE, "vramc_rans.h")]
+SOURCES = [os.path.join(CSRC, f) for f in ("rans_gemv.hip", "rans_decode.hip", "ref32_gemv.hip",
+                                           "w64_host.cpp")]
+HEADERS = [os.path.join(INCLUDE, "vramc_rans.h"), os.path.join(CSRC, "rans_device.h")]
 
 SCALE_BITS = 12
 M = 1 << SCALE_BITS
@@ -53,7 +54,7 @@ SUPPORTED_R = (35, 16, 8, 4, 3, 2, 1)
 LARGE_R = (20,)
 ONE_STATE_R = (35,) + LARGE_R
 
-HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC", "-shared",
+HIPCC_FLAGS = ["-O3", "-std=c++17", "-fPIC",
                # packed fp32 VALU ops stay disabled on this platform
                "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 
@@ -85,10 +86,19 @@ EXPORTS = ("rans_w64_gemv", "rans_w64_gemv_noalloc", "rans_gemv_workspace_bytes"
 
 
 def compile_lib(arch="gfx950", out=LIB):
-    """Compile librans_hip.so with hipcc for ``arch`` (always recompiles)."""
+    """Compile librans_hip.so with hipcc for ``arch`` (always recompiles),
+    one process per source file."""
     tmp = out + ".tmp"
-    cmd = ["hipcc", f"--offload-arch={arch}", *HIPCC_FLAGS, "-o", tmp, *SOURCES]
-    subprocess.check_call(cmd, stderr=subprocess.DEVNULL if os.environ.get("RANS_QUIET") else None)
+    hipcc = ["hipcc", f"--offload-arch={arch}", *HIPCC_FLAGS]
+    err = subprocess.DEVNULL if os.environ.get("RANS_QUIET") else None
+    with tempfile.TemporaryDirectory() as work:
+        objs = [os.path.join(work, os.path.basename(s) + ".o") for s in SOURCES]
+        procs = [subprocess.Popen([*hipcc, "-c", "-o", o, s], stderr=err)
+                 for o, s in zip(objs, SOURCES)]
+        codes = [p.wait() for p in procs]
+        if any(codes):
+            raise subprocess.CalledProcessError(max(codes), hipcc)
+        subprocess.check_call([*hipcc, "-shared", "-o", tmp, *objs], stderr=err)
     os.replace(tmp, out)
     return out
 
