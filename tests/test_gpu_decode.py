@@ -1,0 +1,41 @@
+"""The bf16 and code decode at the sizes where their launches differ: fewer
+and more tiles than one round of waves, tile heights odd and even, below and
+above the size from which rows are stored in pairs, a partial last block of
+column steps, and an output that is only 2-byte aligned."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,cols,R,C,S", [
+    (2050, 256, 1, 64, 1),      # 8200 tiles: several per wave, single rows
+    (4100, 2048, 2, 256, 1),    # 16400 tiles
+    (4098, 2112, 3, 192, 1),    # odd tile height, three column steps per tile
+    (8960, 960, 35, 192, 1),    # one round, odd tile height
+    (4112, 2048, 16, 512, 2),   # two states per lane
+    (2048, 4224, 8, 1408, 1),   # 22 column steps: five blocks and a partial one
+    (4096, 2048, 4, 512, 4),    # four states per lane
+    (32775, 2112, 3, 704, 1),   # 69M weights: paired rows, odd tile height
+    (24, 160, 8, 192, 1),       # one wave, appended columns
+])
+def test_decode_launches(rans, lib, rows, cols, R, C, S):
+    print(f"case decode {rows}x{cols} R={R} C={C} S={S}", flush=True)
+    rng = np.random.default_rng(rows + cols)
+    few = min(rows, 3 * R + 1)  # rows of codes, repeated over the height
+    codes = np.rint(rng.laplace(size=(few, cols)) * 2).astype(np.int32)
+    hit = rng.random(codes.shape) < 0.003
+    codes[hit] = rng.integers(-900, 900, int(hit.sum()))
+    codes = np.resize(codes, (rows, cols))
+    step = (rng.random(cols) + 0.25).astype(np.float32)
+    m = rans.RansMatrix(rans.encode(codes, R, C, S), torch.from_numpy(step), lib)
+    want = (torch.from_numpy(codes).float() * torch.from_numpy(step)).bfloat16().cuda()
+    n = rows * cols
+    for shift in (0, 1, 2, 3):  # of the output, in elements
+        buf = torch.full((n + 8,), 7.0, device="cuda", dtype=torch.bfloat16)
+        out = m.decode(buf[shift:shift + n].view(rows, cols))
+        assert torch.equal(out, want), shift
+        rest = torch.cat([buf[:shift], buf[shift + n:]])
+        assert bool((rest == 7.0).all()), "stored outside the output"
+    np.testing.assert_array_equal(m.decode_codes().cpu().numpy(), codes)

@@ -3,7 +3,9 @@
 // include/vramc_rans.h, the decode step in rans_device.h.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
+#include <type_traits>
 
 #include "../../include/vramc_rans.h"
 #include "rans_device.h"
@@ -11,7 +13,9 @@
 namespace {
 
 // Waves of a decode workgroup (tiles are taken linearly, any count works).
-constexpr int kMaxDecodeWaves = 10;
+constexpr int kMaxDecodeWaves = 16;
+constexpr int64_t kPairWeights = 64 << 20;
+constexpr int kNonTemporal = 2;  // cache policy of a raw buffer store
 constexpr int kDecodeStaticLds = (int)sizeof(TabEntry<false>) * (int)kProbM;
 
 struct DecodeArgs {
@@ -31,13 +35,44 @@ struct DecodeArgs {
     WaveLayout L;
 };
 
+// v of the lane that quad_perm CTRL pairs with this one.
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_swap(uint32_t v) {
+    return __builtin_amdgcn_update_dpp(0u, v, CTRL, 0xF, 0xF, true);
+}
+
 // Decode only.  MODE 0 writes int32 codes, MODE 1 writes bf16(code*step[c]).
-// One wave per tile, the staging and decode step of the GEMV.  Output goes
-// through one buffer resource over the tile row's R output rows: a store's
-// row is its scalar offset, its column step an immediate.  After its own
-// stores have completed, each wave overwrites the escape positions of its
-// tile (decoded as 0) with their side-table values, so no second launch.
-template <int R, int S, int MODE>
+// One wave per tile at a time, the staging and decode step of the GEMV.
+// Output goes through one buffer resource over the tile row's R output rows:
+// a store's row is its scalar offset, its column step an immediate.  Once
+// its own stores have completed, each wave overwrites the escape positions of
+// its tile (decoded as 0) with their side-table values, so no second launch.
+//
+// What bounds a large decode is its writes: storing into a window of 16 tile
+// rows, which stays in the caches, 25600x5120 takes 58 us instead of 100, and
+// writing the same bytes without decoding about 50.  So a bf16 output that
+// takes more than half of the 256 MB memory-side cache (kPairWeights) goes
+// out in
+//   - PAIR: one 4-byte store for two rows.  Lanes l and l^1 hold neighbouring
+//     columns, so they exchange halves and the even lane stores both columns
+//     of the first row, the odd lane both of the second: half the store
+//     instructions, for two more VALU instructions per pair;
+//   - non-temporal stores, which keep the caches for the coded input.
+// 25600x5120 100.2 -> 89.8 us, 5120x25600 113.2 -> 97.5, 34816x5120 104 -> 95.
+// (Pairs alone change nothing, and pairs of column steps or stores of 512
+// contiguous bytes over 4 of them ran slower.)  Smaller outputs are stored
+// plainly: non-temporal stores make those decodes up to 12% faster too, but a
+// matrix product that reads the output next then finds it in HBM instead of
+// the cache (decode and product with 32 rows of x at 5120x5120: 36.0 against
+// 30.9 us, 8960x1536 and 512 rows 35.5 against 32.6; at 13824x5120, 141 MB,
+// and 64 rows 74.2 against 79.4).
+//
+// LOOP: workgroups stay, one per CU; each wave takes tiles first, first +
+// stride, ... and copies the next tile's block as soon as it has decoded the
+// last, so the table is copied once per CU and a wave waits for no other.
+// 5120x5120 in 8x1024 tiles (3200 of them, formerly in workgroups of one
+// wave, 4 waves on a CU) 37.7 -> 19 us.
+template <int R, int S, int MODE, bool PAIR, bool LOOP>
 __global__ void __launch_bounds__(64 * kMaxDecodeWaves) rans_w64_decode_kernel(DecodeArgs a) {
     __shared__ __align__(16) TabEntry<false> tab[kProbM];
     extern __shared__ __align__(16) uint16_t dyn[];
@@ -48,146 +83,230 @@ __global__ void __launch_bounds__(64 * kMaxDecodeWaves) rans_w64_decode_kernel(D
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: scalar tile math
     const int lane = threadIdx.x & 63;
     uint16_t* raw = dyn + (size_t)wave * a.L.wave_words;
-    const int t = blockIdx.x * W + wave;
-    const bool active = t < a.ntiles;
-    const int tc = active ? t : a.ntiles - 1;
-    const int rb = tc / a.ncb, cb = tc - rb * a.ncb;
     asm volatile("" ::"s"(a.tile_off), "s"(a.tile_meta), "s"(a.slen), "s"(a.table_lds),
                  "s"(a.words), "s"(a.step), "s"(a.esc_tileptr), "s"(a.out), "s"(a.C),
                  "s"(a.cols), "s"(a.L.raw_words), "s"(a.W), "s"(a.ncb), "s"(a.ntiles));
+    // LOOP: tiles spread over the workgroups first, so that a last, partial
+    // round leaves every CU with about as many waves; otherwise a workgroup's
+    // tiles are neighbours, whose blocks are too
+    const int stride = gridDim.x * W;
+    int t = LOOP ? wave * gridDim.x + blockIdx.x : blockIdx.x * W + wave;
+    const bool any = t < a.ntiles;
 
-    const TileOff to = load_tile_off(a.tile_off, tc);
-    const int tp = a.esc_tileptr[tc + min(lane, 1)];
-    asm volatile("" ::: "memory");  // keep these two loads first
-    const uint32_t tmv = a.tile_meta[tc];
-    uint32_t len0[S];
+    // what a tile needs from memory besides its block: extent, side-table
+    // range, meta word, lengths; held for the tile in hand and the next one
+    struct Head {
+        TileOff to;
+        int tp;
+        uint32_t tmv, len[S];
+    };
+    auto load_head = [&](int tile) {
+        Head h;
+        const int tc = min(tile, a.ntiles - 1);
+        h.to = load_tile_off(a.tile_off, tc);
+        h.tp = a.esc_tileptr[tc + min(lane, 1)];
+        h.tmv = a.tile_meta[tc];
 #pragma unroll
-    for (int s = 0; s < S; s++) len0[s] = a.slen[tc * nst + 64 * s + lane];
+        for (int s = 0; s < S; s++) h.len[s] = a.slen[tc * nst + 64 * s + lane];
+        return h;
+    };
     const int nk = a.C / nst;
-    const int colbase = cb * a.C + lane;
     const __amdgpu_buffer_rsrc_t srs =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(a.step), 0, a.cols * 4, kBufWord3);
-    float sr[KU][S];
-    auto load_steps = [&](int k0) {
-        const int c0 = colbase + 64 * S * k0;
+    float sr[KU][S];  // steps of the next block of column steps
+    auto load_steps = [&](int c0) {
 #pragma unroll
         for (int u = 0; u < KU; u++)
 #pragma unroll
             for (int s = 0; s < S; s++)
-                sr[u][s] = __uint_as_float(
-                    __builtin_amdgcn_raw_buffer_load_b32(srs, (c0 + 64 * (S * u + s)) * 4, 0, 0));
+                sr[u][s] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+                    srs, (c0 + 64 * (S * u + s)) * 4, 0, 0));
     };
-    if (MODE == 1) load_steps(0);
+    Head cur = load_head(t), next = cur;
+    if constexpr (LOOP) next = load_head(t + stride);
+    if (MODE == 1) load_steps(t % a.ncb * a.C + lane);
     uint32_t o0, n16;
-    tile_extent(to, active, a.L.raw_words, o0, n16);
+    tile_extent(cur.to, any, a.L.raw_words, o0, n16);
     stage_tile(raw, a.words, o0, n16, lane);
     stage_table(tab, a.table_lds, wave, W, lane);
     wait_vm();
     __syncthreads();
-    if (!active) return;
 
-    uint8_t* obase = static_cast<uint8_t*>(a.out) + (size_t)rb * R * a.cols * ESZ;
-    const __amdgpu_buffer_rsrc_t ors =
-        __builtin_amdgcn_make_buffer_rsrc(obase, 0, R * a.cols * ESZ, kBufWord3);
-    Lanes<S, TabEntry<false>> L;
-    uint32_t off0[S], bit0[S], st0[S];
-    stream_layout<S>(len0, __builtin_amdgcn_readfirstlane(tmv), off0, bit0);
+    const bool odd = lane & 1;
+    const uint32_t sel = odd ? 0x03020706u : 0x05040100u;
+    while (t < a.ntiles) {  // wave-uniform
+        const int rb = t / a.ncb, cb = t - rb * a.ncb;
+        const int colbase = cb * a.C + lane;
+        const int e_lo = __builtin_amdgcn_readlane(cur.tp, 0), e_hi = __builtin_amdgcn_readlane(cur.tp, 1);
+        uint8_t* obase = static_cast<uint8_t*>(a.out) + (size_t)rb * R * a.cols * ESZ;
+        const __amdgpu_buffer_rsrc_t ors =
+            __builtin_amdgcn_make_buffer_rsrc(obase, 0, R * a.cols * ESZ, kBufWord3);
+        Lanes<S, TabEntry<false>> L;
+        uint32_t off0[S], bit0[S], st0[S];
+        stream_layout<S>(cur.len, __builtin_amdgcn_readfirstlane(cur.tmv), off0, bit0);
 #pragma unroll
-    for (int s = 0; s < S; s++) st0[s] = initial_state(raw, bit0[s], len0[s]);
-    init_lanes(L, tab, raw, st0, off0);
-    // One block of nu <= KU column steps.  The loop below runs whole blocks
-    // only (nu = KU, no early exit): exits after 1, 2 or 3 steps' stores
-    // would meet at the loop latch, and the compiler would then wait there
-    // for the stores of the longest path.  A partial last block follows it.
-    auto run_block = [&](int k0, int nu) {
-        float sv[KU][S];
-        if (MODE == 1) {
+        for (int s = 0; s < S; s++) st0[s] = initial_state(raw, bit0[s], cur.len[s]);
+        init_lanes(L, tab, raw, st0, off0);
+        // One block of NU <= KU column steps, i.e. NG column groups of 64.  The
+        // loop below runs whole blocks only (no early exit): exits after 1, 2
+        // or 3 steps' stores would meet at the loop latch, and the compiler
+        // would then wait there for the stores of the longest path.  A partial
+        // last block follows it.
+        auto run_block = [&](int k0, auto nu_) {
+            constexpr int NU = decltype(nu_)::value;
+            float sv[KU][S];
+            if (MODE == 1) {
 #pragma unroll
-            for (int u = 0; u < KU; u++)
+                for (int u = 0; u < KU; u++)
 #pragma unroll
-                for (int s = 0; s < S; s++) {
-                    asm volatile("" : "+v"(sr[u][s]));
-                    sv[u][s] = sr[u][s];
-                }
-            // unconditional: past the last block these read columns of the
-            // next tile, or 0 past the end of the matrix, and go unused.  A
-            // conditional prefetch merges two wait states at the join, and
-            // the compiler then waits for this block's stores as well
-            // (vmcnt counts stores too), once per block
-            load_steps(k0 + KU);
-            asm volatile("" ::: "memory");
-        }
-        const int vb = (colbase + 64 * S * k0) * ESZ;
+                    for (int s = 0; s < S; s++) {
+                        asm volatile("" : "+v"(sr[u][s]));
+                        sv[u][s] = sr[u][s];
+                    }
+                // unconditional: past the last block these read columns of the
+                // next tile, or 0 past the end of the matrix, and go unused.  A
+                // conditional prefetch merges two wait states at the join, and
+                // the compiler then waits for this block's stores as well
+                // (vmcnt counts stores too), once per block
+                load_steps(colbase + nst * (k0 + KU));
+                asm volatile("" ::: "memory");
+            }
+            const int vb = (colbase + nst * k0) * ESZ;
+            // paired stores: the lane pair's first column, in odd lanes one
+            // row further down
+            const int vp = vb - 2 * (lane & 1) + (odd ? a.cols * 2 : 0);
 #pragma unroll
-        for (int u = 0; u < KU; u++) {
-            if (u >= nu) break;
+            for (int u = 0; u < NU; u++) {
+                float held[S];
 #pragma unroll
-            for (int r = 0; r < R; r++) {
+                for (int r = 0; r < R; r++) {
 #pragma unroll
-                for (int s = 0; s < S; s++) {
-                    // symbol order within a state is k-major, r-minor, as in the GEMV
-                    const int32_t code = rans_step<(R >= 8)>(L.st[s], L.a[s], L.w[s], L.e[s], tab);
-                    const int vo = vb + 64 * (S * u + s) * ESZ;
-                    if (MODE == 0)
-                        __builtin_amdgcn_raw_buffer_store_b32(code, ors, vo, r * a.cols * 4, 0);
-                    else
-                        __builtin_amdgcn_raw_buffer_store_b16(to_bf16((float)code * sv[u][s]), ors,
-                                                              vo, r * a.cols * 2, 0);
+                    for (int s = 0; s < S; s++) {
+                        // symbol order within a state is k-major, r-minor, as in the GEMV
+                        const int32_t code = rans_step<(R >= 8)>(L.st[s], L.a[s], L.w[s], L.e[s], tab);
+                        const int vo = 64 * (S * u + s) * ESZ;
+                        if constexpr (MODE == 0) {
+                            __builtin_amdgcn_raw_buffer_store_b32(code, ors, vb + vo, r * a.cols * 4, 0);
+                        } else {
+                            const float v = (float)code * sv[u][s];
+                            if (!PAIR || (r == R - 1 && R % 2)) {
+                                __builtin_amdgcn_raw_buffer_store_b16(to_bf16(v), ors, vb + vo,
+                                                                      r * a.cols * 2, PAIR ? kNonTemporal : 0);
+                            } else if (r % 2 == 0) {
+                                held[s] = v;
+                            } else {
+                                const uint32_t p = to_bf16x2(held[s], v);
+                                __builtin_amdgcn_raw_buffer_store_b32(
+                                    __builtin_amdgcn_perm(quad_swap<0xB1>(p), p, sel), ors, vp + vo,
+                                    (r - 1) * a.cols * 2, kNonTemporal);
+                            }
+                        }
+                    }
                 }
             }
+        };
+        const int nk_full = nk - nk % KU;
+        for (int k0 = 0; k0 < nk_full; k0 += KU) run_block(k0, std::integral_constant<int, KU>());
+        switch (nk - nk_full) {
+            case 1: run_block(nk_full, std::integral_constant<int, 1>()); break;
+            case 2: if constexpr (KU > 2) run_block(nk_full, std::integral_constant<int, 2>()); break;
+            case 3: if constexpr (KU > 2) run_block(nk_full, std::integral_constant<int, 3>()); break;
+            default: break;
         }
-    };
-    const int nk_full = nk - nk % KU;
-    for (int k0 = 0; k0 < nk_full; k0 += KU) run_block(k0, KU);
-    if (nk_full < nk) run_block(nk_full, nk - nk_full);
 
-    // Escapes of this tile: its own side-table entries, written over the 0
-    // each escape position was decoded as.  The wave's own stores complete
-    // first, so the value lands after that 0.  Positions are clamped into
-    // the tile, so no side-table content can address outside the output.
-    if (!a.has_esc) return;
-    wait_vm();
-    const int e_lo = __builtin_amdgcn_readlane(tp, 0), e_hi = __builtin_amdgcn_readlane(tp, 1);
-    const int cbase = cb * a.C;
-    for (int e = e_lo + lane; e < e_hi; e += 64) {
-        const int pos = a.esc_pos[e];
-        const int r = esc_row<R>(pos);
-        const int col = cbase + (int)min(esc_tcol<R>(pos), (uint32_t)(a.C - 1));
-        const int32_t v = a.esc_val[e];
-        if (MODE == 0)
-            __builtin_amdgcn_raw_buffer_store_b32(v, ors, (r * a.cols + col) * 4, 0, 0);
-        else
-            __builtin_amdgcn_raw_buffer_store_b16(to_bf16((float)v * a.step[col]), ors,
-                                                  (r * a.cols + col) * 2, 0, 0);
+        // The next tile's block into the wave's region, whose last word has
+        // been read (its LDS reads have returned), its first steps and the
+        // head of the tile after it, in flight together with this tile's
+        // stores.  They are waited for here:
+        // a load pending at the loop's entry would make every block wait for
+        // the stores before it.
+        const int tn = t + stride;
+        Head after = next;
+        if (LOOP && tn < a.ntiles) {  // wave-uniform
+            __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
+            tile_extent(next.to, true, a.L.raw_words, o0, n16);
+            stage_tile(raw, a.words, o0, n16, lane);
+            after = load_head(tn + stride);
+            if (MODE == 1) load_steps(tn % a.ncb * a.C + lane);
+        } else if (!a.has_esc) {
+            return;
+        }
+        wait_vm();
+        // Escapes of this tile: its own side-table entries, written over the 0
+        // each escape position was decoded as.  The wave's own stores have
+        // completed, so the value lands after that 0.  Positions are clamped into
+        // the tile, so no side-table content can address outside the output.
+        if (a.has_esc) {
+            const int cbase = cb * a.C;
+            for (int e = e_lo + lane; e < e_hi; e += 64) {
+                const int pos = a.esc_pos[e];
+                const int r = esc_row<R>(pos);
+                const int col = cbase + (int)min(esc_tcol<R>(pos), (uint32_t)(a.C - 1));
+                const int32_t v = a.esc_val[e];
+                if (MODE == 0)
+                    __builtin_amdgcn_raw_buffer_store_b32(v, ors, (r * a.cols + col) * 4, 0, 0);
+                else
+                    __builtin_amdgcn_raw_buffer_store_b16(to_bf16((float)v * a.step[col]), ors,
+                                                          (r * a.cols + col) * 2, 0, 0);
+            }
+        }
+        if (!LOOP) return;
+        cur = next;
+        next = after;
+        t = tn;
     }
 }
 
-// Waves per decode workgroup: among the counts whose LDS fits, the one that
-// puts the fewest waves on the busiest CU when the workgroups spread evenly
-// over the CUs, the largest such (fewer table copies).
-int decode_waves(const rans_w64_matrix* m) {
+// Waves per decode workgroup when one workgroup per CU takes all the tiles
+// (loop): as many as the LDS holds, but no more than give every wave the same
+// number of tiles.  Otherwise (int32 codes, whose time is their writes), of
+// the counts that put the fewest waves on the busiest CU when the workgroups
+// spread evenly the largest, from 4 up: workgroups of fewer waves fill the
+// LDS with tables.
+int decode_waves(const rans_w64_matrix* m, int64_t ntiles, int cus, bool loop) {
     const WaveLayout L = wave_layout(m);
-    const int64_t ntiles = (int64_t)(m->rows / m->R) * (m->cols / m->C);
-    const int cus = device_cus();
+    int most = 0;
+    while (most < kMaxDecodeWaves && lds_bytes(most + 1, L) + kDecodeStaticLds <= (size_t)kLdsMax)
+        most++;
+    if (!most) return 0;
+    if (loop) {
+        const int64_t rounds = (ntiles + (int64_t)cus * most - 1) / ((int64_t)cus * most);
+        return (int)((ntiles + cus * rounds - 1) / (cus * rounds));
+    }
     int best = 0;
     int64_t best_load = 0;
-    for (int w = 1; w <= kMaxDecodeWaves; w++) {
-        if (lds_bytes(w, L) + kDecodeStaticLds > (size_t)kLdsMax) break;
+    for (int w = std::min(4, most); w <= std::min(10, most); w++) {
         const int64_t grid = (ntiles + w - 1) / w;
-        const int64_t load = cus > 0 ? (grid + cus - 1) / cus * w : -w;
+        const int64_t load = (grid + cus - 1) / cus * w;
         if (!best || load <= best_load) best = w, best_load = load;
     }
     return best;
 }
 
-template <int R, int S, int MODE>
-int launch_decode_t(const DecodeArgs& a, int waves, size_t lds, int grid, hipStream_t stream) {
-    const void* fn = reinterpret_cast<const void*>(&rans_w64_decode_kernel<R, S, MODE>);
+template <int R, int S, int MODE, bool PAIR, bool LOOP>
+int launch_decode_p(const DecodeArgs& a, int waves, size_t lds, int grid, hipStream_t stream) {
+    const void* fn = reinterpret_cast<const void*>(&rans_w64_decode_kernel<R, S, MODE, PAIR, LOOP>);
     hipError_t e = ensure_lds(fn, lds, kDecodeStaticLds);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((rans_w64_decode_kernel<R, S, MODE>), dim3(grid), dim3(64 * waves), lds,
-                       stream, a);
+    hipLaunchKernelGGL((rans_w64_decode_kernel<R, S, MODE, PAIR, LOOP>), dim3(grid), dim3(64 * waves),
+                       lds, stream, a);
     return (int)hipGetLastError();
+}
+
+template <int R, int S, int MODE>
+int launch_decode_t(const DecodeArgs& a, int waves, size_t lds, int grid, hipStream_t stream) {
+    if constexpr (MODE == 1) {
+        const bool loop = (int64_t)grid * waves < a.ntiles;
+        // paired rows in 4-byte stores (rows are a multiple of 128 bytes: cols
+        // is one of 64)
+        if constexpr (R > 1) {
+            if ((uintptr_t)a.out % 4 == 0 && (int64_t)a.rows * a.cols >= kPairWeights)
+                return loop ? launch_decode_p<R, S, MODE, true, true>(a, waves, lds, grid, stream)
+                            : launch_decode_p<R, S, MODE, true, false>(a, waves, lds, grid, stream);
+        }
+        if (loop) return launch_decode_p<R, S, MODE, false, true>(a, waves, lds, grid, stream);
+    }
+    return launch_decode_p<R, S, MODE, false, false>(a, waves, lds, grid, stream);
 }
 
 template <int MODE>
@@ -208,7 +327,10 @@ int launch_decode_common(const rans_w64_matrix* m, void* out, hipStream_t stream
     if (!valid_geometry(m)) return RANS_EGEOMETRY;
     if (!valid_pointers(m) || !out) return RANS_EARG;
     if (!supported_rs(m->R, m->S)) return RANS_EUNSUPPORTED;
-    const int waves = decode_waves(m);
+    const int64_t ntiles = (int64_t)(m->rows / m->R) * (m->cols / m->C);
+    const int cus = device_cus();
+    if (cus <= 0) return (int)hipErrorInvalidDevice;
+    const int waves = decode_waves(m, ntiles, cus, MODE == 1);
     if (!waves) return RANS_EGEOMETRY;
     DecodeArgs a;
     a.words = m->words;
@@ -225,11 +347,12 @@ int launch_decode_common(const rans_w64_matrix* m, void* out, hipStream_t stream
     a.cols = m->cols;
     a.C = m->C;
     a.ncb = m->cols / m->C;
-    a.ntiles = (m->rows / m->R) * a.ncb;
+    a.ntiles = (int)ntiles;
     a.W = waves;
     a.has_esc = !(m->flags & RANS_F_NO_ESCAPES);
     a.L = wave_layout(m);
-    const int grid = (a.ntiles + waves - 1) / waves;
+    const int64_t groups = (ntiles + waves - 1) / waves;
+    const int grid = (int)(MODE == 1 ? std::min<int64_t>(cus, groups) : groups);
     return dispatch_decode<MODE>(a, m->R, m->S, waves, lds_bytes(waves, a.L), grid, stream);
 }
 

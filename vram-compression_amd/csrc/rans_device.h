@@ -360,6 +360,13 @@ __device__ __forceinline__ void lds_add(float* p, float v) {
 // bf16 of f, round to nearest even (gfx950's v_cvt_pk_bf16_f32).
 __device__ __forceinline__ uint16_t to_bf16(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
+// bf16 of lo and hi in the two halves of a word (one v_cvt_pk_bf16_f32).
+__device__ __forceinline__ uint32_t to_bf16x2(float lo, float hi) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
+}
+
 // ------------------------------------------------------------------ host
 WaveLayout wave_layout(const rans_w64_matrix* m) {
     WaveLayout L;
