@@ -70,6 +70,7 @@ extern "C" {
 /* x dtype codes for rans_w64_gemv */
 #define RANS_X_F32 0
 #define RANS_X_BF16 1
+#define RANS_X_F16 2 /* output of rans_linear_finish only */
 
 /* rejected-argument return values */
 #define RANS_EUNSUPPORTED (-1) /* R, S or batch without a compiled kernel: the GPU entry
@@ -194,6 +195,14 @@ int rans_w64_gemv_noalloc(const rans_w64_matrix* m, const void* x, int x_dtype, 
  * are bitwise those of separate rans_w64_gemv calls. */
 int rans_w64_gemv_group(const rans_w64_matrix* const* ms, int n, const void* x, int x_dtype,
                         int batch, float* const* ys, hipStream_t stream);
+
+/* The last pass of a linear layer: out[r,c] = cast(float(y[r*ld + c]) +
+ * bias[c]), one rounding to out_dtype (RANS_X_F32, RANS_X_BF16 or RANS_X_F16).
+ * y is rows x cols (f32 or bf16) with ld >= cols values from row to row, out is
+ * contiguous, bias is f32 or NULL.  RANS_EARG for null pointers, sizes or
+ * types outside these.  No reference counterpart. */
+int rans_linear_finish(const void* y, int y_dtype, int64_t ld, const float* bias, void* out,
+                       int out_dtype, int64_t rows, int cols, hipStream_t stream);
 
 /* Decode to a dense bf16 matrix out[r,c] = bf16(code[r,c]*step[c]) (round to
  * nearest even).  Replaces launch_rans_decode (rans_gemv.cu:155-162). */

@@ -26,8 +26,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "librans_hip.so")
-SOURCES = [os.path.join(CSRC, f) for f in ("rans_gemv.hip", "rans_decode.hip", "ref32_gemv.hip",
-                                           "w64_host.cpp")]
+SOURCES = [os.path.join(CSRC, f) for f in ("rans_gemv.hip", "rans_decode.hip", "rans_linear.hip",
+                                           "ref32_gemv.hip", "w64_host.cpp")]
 HEADERS = [os.path.join(INCLUDE, "vramc_rans.h"), os.path.join(CSRC, "rans_device.h")]
 
 SCALE_BITS = 12
@@ -37,7 +37,7 @@ OFFSET = 128
 ESC = 0  # escape symbol: codes outside [-127, 127]
 LANES = 64
 
-X_F32, X_BF16 = 0, 1
+X_F32, X_BF16, X_F16 = 0, 1, 2
 # stream layouts, recorded as enc["layout"]: the wavefront-interleaved w64
 # format of `encode`, and the reference's own 32-lane format
 # (encode_reference_layout, or the reference's encode itself)
@@ -77,7 +77,7 @@ class RansMatrixDesc(ctypes.Structure):
 EXPORTS = ("rans_w64_gemv", "rans_w64_gemv_noalloc", "rans_gemv_workspace_bytes", "rans_gemv_table4",
            "rans_gemv_rows2", "rans_w64_gemv_group", "launch_rans_gemv", "launch_rans_decode",
            "rans_w64_decode",
-           "rans_w64_decode_codes", "launch_int4_gemv", "bf16_gemv", "rans_build_table",
+           "rans_w64_decode_codes", "rans_linear_finish", "launch_int4_gemv", "bf16_gemv", "rans_build_table",
            "rans_table_lds",
            "rans_table_lds4",
            "rans_w64_encode", "rans_w64_encode_fetch", "rans_w64_encode_counts",
@@ -130,6 +130,8 @@ def load_lib(path=LIB):
         "launch_rans_decode": ([ctypes.c_int] + [P] * 5 + [ctypes.c_int] * 3 + [P], ctypes.c_int),
         "rans_w64_decode": ([D, P, P], ctypes.c_int),
         "rans_w64_decode_codes": ([D, P, P], ctypes.c_int),
+        "rans_linear_finish": ([P, ctypes.c_int, I64, P, P, ctypes.c_int, I64, ctypes.c_int, P],
+                               ctypes.c_int),
         "launch_int4_gemv": ([P, P, P, ctypes.c_int, ctypes.c_int, P], ctypes.c_int),
         "bf16_gemv": ([P, P, P, ctypes.c_int, ctypes.c_int, P], ctypes.c_int),
         "rans_build_table": ([P, I64, P, P, P], ctypes.c_int),
@@ -587,6 +589,24 @@ def fused_rows_limit(desc, lib, grouped=False):
 
 
 # ------------------------------------------------------------------- device
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
+def _device():
+    """Index of the current device."""
+    return torch.cuda.current_device() if _current_device is None else _current_device()
+
+
+def _stream():
+    """The current stream's handle.  torch.cuda.current_stream() wraps it in
+    a Python object, at 2.7 us a call a quarter of a small GEMV's host time;
+    the handle itself takes 0.2."""
+    if _raw_stream is None or _current_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
+
+
 def _require_gpu():
     if not torch.cuda.is_available():
         raise RuntimeError("RansMatrix needs a ROCm GPU (gfx950); no CPU fallback exists")

@@ -21,6 +21,7 @@ import weakref
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 import rans
 
@@ -58,6 +59,42 @@ def quantize_uniform(weight, bits, iters=40, sample=1 << 22, seed=0):
     return codes, np.full(w.shape[1], delta, np.float32)
 
 
+_DTYPES = {torch.float32: rans.X_F32, torch.bfloat16: rans.X_BF16, torch.float16: rans.X_F16}
+_peek_functorch = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack",
+                          lambda: None)
+
+
+def _plain(t):
+    """Whether t is an ordinary tensor of the current GPU that nothing else
+    watches: no gradient, forward-mode, vmap, tracing or dispatch mode that an
+    operation outside torch would be hidden from."""
+    return (type(t) is torch.Tensor and t.is_cuda and not t.requires_grad
+            and t.get_device() == rans._device() and not torch.compiler.is_compiling()
+            and forward_ad._current_level < 0 and _peek_functorch() is None
+            and torch._C._get_tracing_state() is None
+            and torch._C._len_torch_dispatch_stack() == 0)
+
+
+def _finish(lib, y, bias, dtype):
+    """(y.float() + bias).to(dtype) for a product y (rows x out_features, f32
+    or bf16, rows possibly wider apart): one pass (rans_linear_finish) where y
+    is a plain tensor, the same torch operations otherwise, bitwise alike."""
+    if bias is None and y.dtype is dtype and y.is_contiguous():
+        return y
+    rows, cols = y.shape
+    if (rows and y.stride(1) == 1 and (rows == 1 or y.stride(0) >= cols) and _plain(y)
+            and (bias is None or (_plain(bias) and bias.dtype is torch.float32
+                                  and bias.dim() == 1 and bias.is_contiguous()))):
+        out = torch.empty((rows, cols), device=y.device, dtype=dtype)
+        rc = lib.rans_linear_finish(y.data_ptr(), _DTYPES[y.dtype], max(y.stride(0), cols),
+                                    None if bias is None else bias.data_ptr(), out.data_ptr(),
+                                    _DTYPES[dtype], rows, cols, rans._stream())
+        assert rc == 0, f"HIP error {rc}"
+        return out
+    y = y.float()
+    return (y if bias is None else y + bias).to(dtype)
+
+
 class LinearGroup:
     """RansLinear modules that read the same input: a decoder layer's q, k
     and v projections, or its gate and up.  When a member is called, every
@@ -78,7 +115,8 @@ class LinearGroup:
 
     def product(self, member, x, xd):
         """member's x @ W^T (no bias) for the module input x, flattened and
-        converted to xd (rows x in_features, f32 or bf16); f32."""
+        converted to xd (rows x in_features, f32 or bf16); f32, or bf16 from
+        the dense GEMM."""
         i = next(j for j, m in enumerate(self.members) if m is member)
         if (self._x is not None and self._x() is x and self._version == x._version
                 and i in self._pending):
@@ -92,7 +130,7 @@ class LinearGroup:
             for m in self.members:
                 m.matrix.decode(w[off:off + m.out_features])
                 off += m.out_features
-            yall = torch.nn.functional.linear(xd.to(torch.bfloat16), w).float()
+            yall = torch.nn.functional.linear(xd.to(torch.bfloat16), w)
             off = 0
             for m in self.members:
                 ys.append(yall[:, off:off + m.out_features])
@@ -147,21 +185,18 @@ class RansLinear(torch.nn.Module):
         if x.shape[-1] != self.in_features:
             raise ValueError(f"expected last dim {self.in_features}, got {x.shape[-1]}")
         lead = x.shape[:-1]
-        xd = x.reshape(-1, self.in_features)
+        xd = x if x.dim() == 2 else x.reshape(-1, self.in_features)
         if xd.dtype not in (torch.bfloat16, torch.float32):
             xd = xd.float()
         if self.group is not None:
             y = self.group.product(self, x, xd.contiguous())
-        elif xd.shape[0] > self.matrix.fused_rows_limit:
+        elif xd.shape[0] > 8 and xd.shape[0] > self.matrix.fused_rows_limit:
             w = self.matrix.decode()  # bf16 code*step, then the dense GEMM
-            y = torch.nn.functional.linear(xd.to(torch.bfloat16), w).float()
+            y = torch.nn.functional.linear(xd.to(torch.bfloat16), w)
         else:
             y = self.matrix.gemv(xd.contiguous())
-        if self.bias is not None:
-            y = y + self.bias
-        out_dtype = x.dtype if x.dtype in (torch.bfloat16, torch.float16, torch.float32) \
-            else torch.float32
-        return y.to(out_dtype).reshape(*lead, self.out_features)
+        y = _finish(self.matrix.lib, y, self.bias, x.dtype if x.dtype in _DTYPES else torch.float32)
+        return y if len(lead) == 1 else y.reshape(*lead, self.out_features)
 
     def extra_repr(self):
         m = self.matrix
