@@ -589,6 +589,7 @@ def fused_rows_limit(desc, lib, grouped=False):
 
 
 # ------------------------------------------------------------------- device
+_CUDA = torch.device("cuda")
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 _current_device = getattr(torch._C, "_cuda_getDevice", None)
 
@@ -750,28 +751,28 @@ class RansMatrix:
         through a zero-padded copy (the kernel reads stream_cols values per
         x row)."""
         assert x.is_cuda, "x must be a device tensor"
-        squeeze = x.dim() == 1
-        xb = x.reshape(1, -1) if squeeze else x
-        assert xb.shape[-1] == self.cols
-        xb, xd = _x_operand(xb, self.stream_cols)
-        B = xb.shape[0]
+        dim = x.dim()
+        assert x.shape[-1] == self.cols
+        B = 1 if dim == 1 else x.shape[0]
+        x, xd = _x_operand(x, self.stream_cols)
         if y is None:
-            y = torch.empty((B, self.rows) if not squeeze else (self.rows,),
-                            device="cuda", dtype=torch.float32)
-        assert y.dtype == torch.float32 and y.is_contiguous() and y.numel() == B * self.rows
-        rc = self.lib.rans_w64_gemv(ctypes.byref(self._desc), xb.data_ptr(), xd, B,
-                                       y.data_ptr(), torch.cuda.current_stream().cuda_stream)
+            y = torch.empty((B, self.rows) if dim != 1 else (self.rows,),
+                            device=_CUDA, dtype=torch.float32)
+        else:
+            assert y.dtype == torch.float32 and y.is_contiguous() and y.numel() == B * self.rows
+        rc = self.lib.rans_w64_gemv(ctypes.byref(self._desc), x.data_ptr(), xd, B, y.data_ptr(),
+                                    _stream())
         assert rc == 0, f"HIP error {rc}"
         return y
 
     def _decode_into(self, fn, out, dtype):
         if out is None:
-            out = torch.empty(self.rows, self.cols, device="cuda", dtype=dtype)
+            out = torch.empty((self.rows, self.cols), device=_CUDA, dtype=dtype)
         assert out.dtype == dtype and out.is_contiguous() and out.numel() == self.rows * self.cols
         # appended columns: decode the stored width, keep the matrix's own
         full = out if self.stream_cols == self.cols else \
             torch.empty(self.rows, self.stream_cols, device="cuda", dtype=dtype)
-        rc = fn(ctypes.byref(self._desc), full.data_ptr(), torch.cuda.current_stream().cuda_stream)
+        rc = fn(ctypes.byref(self._desc), full.data_ptr(), _stream())
         assert rc == 0, f"HIP error {rc}"
         if full is not out:
             out.view(self.rows, self.cols).copy_(full[:, :self.cols])
@@ -787,6 +788,7 @@ class RansMatrix:
 
 
 GROUP_MAX = 4
+_POINTERS = [ctypes.c_void_p * n for n in range(GROUP_MAX + 1)]
 _EUNSUPPORTED, _EGEOMETRY, _ECODES = -1, -2, -5
 
 
@@ -802,15 +804,18 @@ def pick_group_tiling(rows_list, cols, S=1):
 
 
 def _x_operand(xb, scols):
-    """x rows as the kernels read them: contiguous bf16 or f32, each row
-    zero-padded to scols values (a matrix stored with appended columns)."""
-    if xb.dtype == torch.bfloat16:
+    """x (one vector or rows of them) as the kernels read it: contiguous bf16
+    or f32, each row zero-padded to scols values (a matrix stored with
+    appended columns)."""
+    if xb.dtype is torch.bfloat16:
         xd = X_BF16
     else:
-        xb, xd = xb.float(), X_F32
+        xd = X_F32
+        if xb.dtype is not torch.float32:
+            xb = xb.float()
     if xb.shape[-1] != scols:
         xb = torch.nn.functional.pad(xb, (0, scols - xb.shape[-1]))
-    return xb.contiguous(), xd
+    return (xb if xb.is_contiguous() else xb.contiguous()), xd
 
 
 def gemv_group(matrices, x, ys=None):
@@ -823,26 +828,27 @@ def gemv_group(matrices, x, ys=None):
     assert 0 < len(ms), "no matrices"
     assert x.is_cuda, "x must be a device tensor"
     squeeze = x.dim() == 1
-    xb0 = x.reshape(1, -1) if squeeze else x
-    B = xb0.shape[0]
+    B = 1 if squeeze else x.shape[0]
+    for m in ms:
+        assert x.shape[-1] == m.cols
     if ys is None:
-        ys = [torch.empty((B, m.rows) if not squeeze else (m.rows,), device="cuda",
+        ys = [torch.empty((B, m.rows) if not squeeze else (m.rows,), device=_CUDA,
                           dtype=torch.float32) for m in ms]
-    assert len(ys) == len(ms)
-    for m, y in zip(ms, ys):
-        assert xb0.shape[-1] == m.cols
-        assert y.dtype == torch.float32 and y.is_contiguous() and y.numel() == B * m.rows
-    xb, xd = _x_operand(xb0, ms[0].stream_cols)
+    else:
+        assert len(ys) == len(ms)
+        for m, y in zip(ms, ys):
+            assert y.dtype == torch.float32 and y.is_contiguous() and y.numel() == B * m.rows
+    xb, xd = _x_operand(x, ms[0].stream_cols)
     if 1 < len(ms) <= GROUP_MAX:
-        descs = (ctypes.c_void_p * len(ms))(*[ctypes.addressof(m._desc) for m in ms])
-        yps = (ctypes.c_void_p * len(ms))(*[y.data_ptr() for y in ys])
-        rc = ms[0].lib.rans_w64_gemv_group(descs, len(ms), xb.data_ptr(), xd, B, yps,
-                                              torch.cuda.current_stream().cuda_stream)
+        n = len(ms)
+        rc = ms[0].lib.rans_w64_gemv_group(
+            _POINTERS[n](*[ctypes.addressof(m._desc) for m in ms]), n, xb.data_ptr(), xd, B,
+            _POINTERS[n](*[y.data_ptr() for y in ys]), _stream())
         if rc == 0:
             return ys
         assert rc in (_EUNSUPPORTED, _EGEOMETRY), f"HIP error {rc}"
     for m, y in zip(ms, ys):
-        m.gemv(xb0 if not squeeze else xb0[0], y)
+        m.gemv(x, y)
     return ys
 
 
@@ -910,8 +916,7 @@ class ReferenceLayoutMatrix:
 
     def _call(self, fn, src, dst):
         rc = fn(self.R, self.words.data_ptr(), self.offs.data_ptr(), self.table.data_ptr(),
-                src.data_ptr(), dst.data_ptr(), self.rows, self.cols, self.C,
-                torch.cuda.current_stream().cuda_stream)
+                src.data_ptr(), dst.data_ptr(), self.rows, self.cols, self.C, _stream())
         assert rc == 0, f"HIP error {rc}"
         return dst
 
