@@ -226,3 +226,28 @@ def test_reference_format_unaligned_words(rans, lib, golden, dev):
     ref = O.gemv_f64(codes, x.cpu().numpy().astype(np.float64), np.ones(cols))
     yv = y.cpu().numpy().astype(np.float64)
     assert np.linalg.norm(yv - ref) / np.linalg.norm(ref) <= REL_L2
+
+
+@pytest.mark.parametrize("rows,cols,R,C", [(8, 32, 1, 32), (5, 544, 1, 544), (8, 352, 2, 352),
+                                           (20, 448, 4, 224), (48, 96, 16, 96)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_reference_format_short_blocks(rans, oracle, lib, dev, rows, cols, R, C, shift):
+    """Column steps that 16 symbols ahead do not divide, one to seventeen of
+    them, with the table on and off a 16-byte boundary (shift words)."""
+    print(f"case ref32 {rows}x{cols} R={R} C={C} shift={shift}", flush=True)
+    codes = oracle.synth_codes(rows, cols, 3.0, seed=rows + cols).astype(np.int64)
+    enc = oracle.encode_ref(codes, R, C)
+    words, offs, table = _upload(enc)
+    moved = torch.zeros(4096 + shift, dtype=torch.int32, device="cuda")[shift:]
+    moved.copy_(table)
+    step = torch.full((cols,), 0.5, device="cuda")
+    out = torch.empty(rows, cols, device="cuda", dtype=torch.bfloat16)
+    x = torch.ones(cols, device="cuda")
+    y = torch.zeros(rows, device="cuda")
+    args = words.data_ptr(), offs.data_ptr(), moved.data_ptr()
+    st = torch.cuda.current_stream().cuda_stream
+    assert lib.launch_rans_decode(R, *args, step.data_ptr(), out.data_ptr(), rows, cols, C, st) == 0
+    assert lib.launch_rans_gemv(R, *args, x.data_ptr(), y.data_ptr(), rows, cols, C, st) == 0
+    want = torch.from_numpy(codes).cuda()
+    assert torch.equal(out.float(), want * 0.5)  # |code| <= 128: exact in bf16
+    assert torch.equal(y, want.sum(1).float())   # whole numbers: exact sums

@@ -30,6 +30,8 @@
 // holds `words` (queried on the host): no copy reads outside it.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <mutex>
 
@@ -90,19 +92,27 @@ __device__ __forceinline__ uint16_t ref_bf16(float f) {
 // slot-cum}, software-pipelined: e holds the table entry of this symbol,
 // read in the previous step, and the next entry is read as soon as the new
 // state exists, ahead of the word refill; the next word w is read ahead.
-// Words in LDS: the select form (the read-ahead word is long back when the
-// select needs it).
-__device__ __forceinline__ int32_t ref_step_lds(uint32_t& st, uint32_t& ad, uint32_t& w, uint2& e,
-                                                const uint2* tab) {
+// Words in LDS.  A wave runs its streams nearly alone on a CU, so the time is
+// the length of one step's chain: the table entry's latency plus what stands
+// between its arrival and the next read.  So two words are read ahead, w and
+// w1: with one, each step waited for the word as well as for the entry.  The
+// next slot comes straight from the low bits of state or word (a word has all
+// 12 of them), and everything else waits until its read is out.  1536x8960 in
+// 8x8960 tiles (2240 symbols a stream, 96 waves) 119.8 -> 106.6 us; the same
+// step with one word read ahead on every lane took 143, and half as many
+// lanes per wave, on twice the waves, 128.
+__device__ __forceinline__ int32_t ref_step_lds(uint32_t& st, uint32_t& ad, uint32_t& w,
+                                                uint32_t& w1, uint2& e, const uint2* tab) {
     const uint2 cur = e;
     const uint32_t ns = __umul24(cur.x, st >> 12) + cur.y;
     const bool need = ns < kRefL;
+    e = tab[(need ? w : ns) & (kRefM - 1)];
+    __builtin_amdgcn_sched_barrier(0);
     st = need ? ((ns << 16) | w) : ns;
-    e = tab[st & (kRefM - 1)];
-    if (need) {
-        ad += 2u;
-        w = ref_lds_u16(ad);
-    }
+    w = need ? w1 : w;
+    ad += need ? 2u : 0u;
+    w1 = ref_lds_u16(ad);
+    __builtin_amdgcn_sched_barrier(0);
     return (int32_t)cur.x >> 24;
 }
 
@@ -132,9 +142,26 @@ __global__ void __launch_bounds__(64 * kRefMaxWaves) ref32_kernel(Ref32Args a) {
     const int W = blockDim.x >> 6;
     // the reference's packed table as the 8-byte image; code = sym - 128 for
     // every symbol of this format (it has no escapes)
-    for (int i = threadIdx.x; i < (int)kRefM; i += blockDim.x) {
-        const uint32_t e = a.table[i];
+    auto put = [&](int i, uint32_t e) {
         tab[i] = make_uint2(((e >> 8) & 0xFFFu) | (((e & 0xFFu) - 128u) << 24), e >> 20);
+    };
+    if (((uintptr_t)a.table & 15) == 0) {
+        // four entries a load, four loads in flight: one wave alone fetches
+        // the 16 KB in four round trips
+        const uint4* t4 = reinterpret_cast<const uint4*>(a.table);
+        for (int i = threadIdx.x; i < (int)kRefM / 4; i += 4 * blockDim.x) {
+            uint4 v[4];
+#pragma unroll
+            for (int u = 0; u < 4; u++) v[u] = t4[min(i + u * (int)blockDim.x, (int)kRefM / 4 - 1)];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                const int j = i + u * (int)blockDim.x;
+                if (j >= (int)kRefM / 4) break;
+                put(4 * j, v[u].x), put(4 * j + 1, v[u].y), put(4 * j + 2, v[u].z), put(4 * j + 3, v[u].w);
+            }
+        }
+    } else {
+        for (int i = threadIdx.x; i < (int)kRefM; i += blockDim.x) put(i, a.table[i]);
     }
     const int g = blockIdx.x * W + wave;  // this wave's group of 64 lanes
     const int base = g * 64;
@@ -224,15 +251,29 @@ __global__ void __launch_bounds__(64 * kRefMaxWaves) ref32_kernel(Ref32Args a) {
         if (staged) {
             uint32_t ad = ref_lds_addr(slot + (p0 - (uint32_t)w0));
             uint32_t st = (ref_lds_u16(ad) << 16) | ref_lds_u16(ad + 2u);
-            ad += 4u;
-            uint32_t w = ref_lds_u16(ad);
+            uint32_t w = ref_lds_u16(ad + 4u);
+            ad += 6u;  // of the word after w
+            uint32_t w1 = ref_lds_u16(ad);
             uint2 e = tab[st & (kRefM - 1)];
-            float xn = a.xs[col0];
-            for (int k = 0; k < nk; k++) {
-                const float xv = xn;
-                xn = a.xs[col0 + 32 * min(k + 1, nk - 1)];
+            // x (or the steps) 16 symbols ahead of use: with short tiles one
+            // column step is far less than a load's latency (512x8192 in
+            // 1x8192 tiles 64.9 -> 29.0 us, 8192x1536 in 2x1536 21.0 -> 16.4)
+            constexpr int KU = 16 / R;
+            float xn[KU], xv[KU];
 #pragma unroll
-                for (int r = 0; r < R; r++) emit(k, r, ref_step_lds(st, ad, w, e, tab), xv);
+            for (int u = 0; u < KU; u++) xn[u] = a.xs[col0 + 32 * min(u, nk - 1)];
+            for (int k0 = 0; k0 < nk; k0 += KU) {
+#pragma unroll
+                for (int u = 0; u < KU; u++) xv[u] = xn[u];
+#pragma unroll
+                for (int u = 0; u < KU; u++) xn[u] = a.xs[col0 + 32 * min(k0 + KU + u, nk - 1)];
+#pragma unroll
+                for (int u = 0; u < KU; u++) {
+                    if (k0 + u >= nk) break;
+#pragma unroll
+                    for (int r = 0; r < R; r++)
+                        emit(k0 + u, r, ref_step_lds(st, ad, w, w1, e, tab), xv[u]);
+                }
             }
         } else {
             // ranged from the wave's first offset, so the byte offsets stay
@@ -287,6 +328,19 @@ hipError_t ref_ensure_lds(const void* fn, size_t bytes) {
     return e;
 }
 
+// CUs of the current device, cached per device; 0 when the query fails.
+std::atomic<int> g_ref_cus[64];
+
+int ref_cus() {
+    int dev = 0, cus = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
+    if (dev < 64 && (cus = g_ref_cus[dev].load(std::memory_order_relaxed)) > 0) return cus;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+        return 0;
+    if (dev < 64) g_ref_cus[dev].store(cus, std::memory_order_relaxed);
+    return cus;
+}
+
 template <int R, bool DECODE>
 int ref32_launch(const Ref32Args& a, int W, hipStream_t stream) {
     const void* fn = reinterpret_cast<const void*>(&ref32_kernel<R, DECODE>);
@@ -339,8 +393,12 @@ int ref32_entry(int R, const void* words, const void* offs, const void* table, c
     slot = (slot + 7) / 8 * 8;
     if (slot > kRefSlotMax) slot = kRefSlotMax;
     a.slot = (int)slot;
+    // as many waves as share a table without leaving CUs idle
+    const int cus = ref_cus();
+    const int64_t per_cu = cus > 0 ? ((nlanes + 63) / 64 + cus - 1) / cus : kRefMaxWaves;
     int W = (kRefLdsMax - kRefStaticLds) / (int)(slot * 2);
-    W = W < 1 ? 1 : (W > kRefMaxWaves ? kRefMaxWaves : W);
+    W = (int)std::min<int64_t>(std::min(W, kRefMaxWaves), per_cu);
+    if (W < 1) W = 1;
     switch (R) {
         case 1: return ref32_launch<1, DECODE>(a, W, stream);
         case 2: return ref32_launch<2, DECODE>(a, W, stream);
