@@ -70,7 +70,7 @@ extern "C" {
 /* x dtype codes for rans_w64_gemv */
 #define RANS_X_F32 0
 #define RANS_X_BF16 1
-#define RANS_X_F16 2 /* output of rans_linear_finish only */
+#define RANS_X_F16 2 /* output of rans_linear_finish and rans_w64_matmul only */
 
 /* rejected-argument return values */
 #define RANS_EUNSUPPORTED (-1) /* R, S or batch without a compiled kernel: the GPU entry
@@ -203,6 +203,18 @@ int rans_w64_gemv_group(const rans_w64_matrix* const* ms, int n, const void* x, 
  * types outside these.  No reference counterpart. */
 int rans_linear_finish(const void* y, int y_dtype, int64_t ld, const float* bias, void* out,
                        int out_dtype, int64_t rows, int cols, hipStream_t stream);
+
+/* A product of up to 64 rows of x on the matrix cores, fused with the decode:
+ * out[b,r] = cast(sum_c bf16(code[r,c]*step[c]) * x[b,c] + bias[r]), sums in
+ * f32, one rounding to out_dtype (RANS_X_F32, RANS_X_BF16 or RANS_X_F16).  x is
+ * batch x cols bf16, 16-byte aligned, bias f32 or NULL, out batch x rows.
+ * RANS_EUNSUPPORTED or RANS_EGEOMETRY, before any launch, for a matrix or
+ * batch it does not take.  rans_matmul_rows: the largest batch it takes that
+ * way and is the faster path for, 0 where it is for none (host code, no GPU
+ * needed).  No reference counterpart. */
+int rans_w64_matmul(const rans_w64_matrix* m, const void* x, int batch, const float* bias,
+                    void* out, int out_dtype, hipStream_t stream);
+int rans_matmul_rows(const rans_w64_matrix* m);
 
 /* Decode to a dense bf16 matrix out[r,c] = bf16(code[r,c]*step[c]) (round to
  * nearest even).  Replaces launch_rans_decode (rans_gemv.cu:155-162). */

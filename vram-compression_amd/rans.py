@@ -26,7 +26,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 LIB = os.path.join(HERE, "librans_hip.so")
-SOURCES = [os.path.join(CSRC, f) for f in ("rans_gemv.hip", "rans_decode.hip", "rans_linear.hip",
+SOURCES = [os.path.join(CSRC, f) for f in ("rans_gemv.hip", "rans_decode.hip", "rans_linear.hip", "rans_matmul.hip",
                                            "ref32_gemv.hip", "w64_host.cpp")]
 HEADERS = [os.path.join(INCLUDE, "vramc_rans.h"), os.path.join(CSRC, "rans_device.h")]
 
@@ -38,6 +38,7 @@ ESC = 0  # escape symbol: codes outside [-127, 127]
 LANES = 64
 
 X_F32, X_BF16, X_F16 = 0, 1, 2
+_X_CODES = {torch.float32: X_F32, torch.bfloat16: X_BF16, torch.float16: X_F16}
 # stream layouts, recorded as enc["layout"]: the wavefront-interleaved w64
 # format of `encode`, and the reference's own 32-lane format
 # (encode_reference_layout, or the reference's encode itself)
@@ -77,7 +78,8 @@ class RansMatrixDesc(ctypes.Structure):
 EXPORTS = ("rans_w64_gemv", "rans_w64_gemv_noalloc", "rans_gemv_workspace_bytes", "rans_gemv_table4",
            "rans_gemv_rows2", "rans_w64_gemv_group", "launch_rans_gemv", "launch_rans_decode",
            "rans_w64_decode",
-           "rans_w64_decode_codes", "rans_linear_finish", "launch_int4_gemv", "bf16_gemv", "rans_build_table",
+           "rans_w64_decode_codes", "rans_linear_finish",
+           "rans_w64_matmul", "rans_matmul_rows", "launch_int4_gemv", "bf16_gemv", "rans_build_table",
            "rans_table_lds",
            "rans_table_lds4",
            "rans_w64_encode", "rans_w64_encode_fetch", "rans_w64_encode_counts",
@@ -132,6 +134,8 @@ def load_lib(path=LIB):
         "rans_w64_decode_codes": ([D, P, P], ctypes.c_int),
         "rans_linear_finish": ([P, ctypes.c_int, I64, P, P, ctypes.c_int, I64, ctypes.c_int, P],
                                ctypes.c_int),
+        "rans_w64_matmul": ([D, P, ctypes.c_int, P, P, ctypes.c_int, P], ctypes.c_int),
+        "rans_matmul_rows": ([D], ctypes.c_int),
         "launch_int4_gemv": ([P, P, P, ctypes.c_int, ctypes.c_int, P], ctypes.c_int),
         "bf16_gemv": ([P, P, P, ctypes.c_int, ctypes.c_int, P], ctypes.c_int),
         "rans_build_table": ([P, I64, P, P, P], ctypes.c_int),
@@ -675,6 +679,8 @@ class RansMatrix:
             step=self.step.data_ptr(), workspace=None, workspace_bytes=0)
         self.workspace = None
         self._ensure_workspace(4)
+        # rows of x up to which matmul beats decoding and a dense product
+        self.matmul_rows = int(lib.rans_matmul_rows(ctypes.byref(self._desc)))
         self.table_lds4 = None
         if flags & F_TABLE4 or (not flags & F_TABLE8 and
                                 lib.rans_gemv_table4(ctypes.byref(self._desc), X_BF16, 1) == 1):
@@ -764,6 +770,21 @@ class RansMatrix:
                                     _stream())
         assert rc == 0, f"HIP error {rc}"
         return y
+
+    def matmul(self, x, bias=None, dtype=torch.float32):
+        """x @ W^T + bias for up to matmul_rows rows of x, the weights rounded
+        to bf16 as decode rounds them and multiplied on the matrix cores with
+        x in bf16, sums in f32 and one rounding to dtype (f32, bf16 or f16)."""
+        assert x.is_cuda and x.dim() == 2 and x.shape[1] == self.cols
+        x, _ = _x_operand(x.to(torch.bfloat16), self.stream_cols)
+        if x.data_ptr() % 16:  # the kernel reads 16 bytes at a time
+            x = x.clone()
+        out = torch.empty((x.shape[0], self.rows), device=_CUDA, dtype=dtype)
+        rc = self.lib.rans_w64_matmul(ctypes.byref(self._desc), x.data_ptr(), x.shape[0],
+                                      None if bias is None else bias.data_ptr(), out.data_ptr(),
+                                      _X_CODES[dtype], _stream())
+        assert rc == 0, f"HIP error {rc}"
+        return out
 
     def _decode_into(self, fn, out, dtype):
         if out is None:

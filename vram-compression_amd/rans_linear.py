@@ -59,7 +59,7 @@ def quantize_uniform(weight, bits, iters=40, sample=1 << 22, seed=0):
     return codes, np.full(w.shape[1], delta, np.float32)
 
 
-_DTYPES = {torch.float32: rans.X_F32, torch.bfloat16: rans.X_BF16, torch.float16: rans.X_F16}
+_DTYPES = rans._X_CODES
 _peek_functorch = getattr(getattr(torch._C, "_functorch", None), "peek_interpreter_stack",
                           lambda: None)
 
@@ -75,6 +75,12 @@ def _plain(t):
             and torch._C._len_torch_dispatch_stack() == 0)
 
 
+def _plain_bias(bias):
+    """Whether bias is None or one the kernels read: plain, f32, contiguous."""
+    return bias is None or (_plain(bias) and bias.dtype is torch.float32 and bias.dim() == 1
+                            and bias.is_contiguous())
+
+
 def _finish(lib, y, bias, dtype):
     """(y.float() + bias).to(dtype) for a product y (rows x out_features, f32
     or bf16, rows possibly wider apart): one pass (rans_linear_finish) where y
@@ -83,8 +89,7 @@ def _finish(lib, y, bias, dtype):
         return y
     rows, cols = y.shape
     if (rows and y.stride(1) == 1 and (rows == 1 or y.stride(0) >= cols) and _plain(y)
-            and (bias is None or (_plain(bias) and bias.dtype is torch.float32
-                                  and bias.dim() == 1 and bias.is_contiguous()))):
+            and _plain_bias(bias)):
         out = torch.empty((rows, cols), device=y.device, dtype=dtype)
         rc = lib.rans_linear_finish(y.data_ptr(), _DTYPES[y.dtype], max(y.stride(0), cols),
                                     None if bias is None else bias.data_ptr(), out.data_ptr(),
@@ -93,6 +98,10 @@ def _finish(lib, y, bias, dtype):
         return out
     y = y.float()
     return (y if bias is None else y + bias).to(dtype)
+
+
+def _out_dtype(x):
+    return x.dtype if x.dtype in _DTYPES else torch.float32
 
 
 class LinearGroup:
@@ -191,11 +200,15 @@ class RansLinear(torch.nn.Module):
         if self.group is not None:
             y = self.group.product(self, x, xd.contiguous())
         elif xd.shape[0] > 8 and xd.shape[0] > self.matrix.fused_rows_limit:
+            if (xd.shape[0] <= self.matrix.matmul_rows and _plain(x) and _plain_bias(self.bias)
+                    and not torch.is_autocast_enabled("cuda")):
+                y = self.matrix.matmul(xd, self.bias, _out_dtype(x))
+                return y if len(lead) == 1 else y.reshape(*lead, self.out_features)
             w = self.matrix.decode()  # bf16 code*step, then the dense GEMM
             y = torch.nn.functional.linear(xd.to(torch.bfloat16), w)
         else:
             y = self.matrix.gemv(xd.contiguous())
-        y = _finish(self.matrix.lib, y, self.bias, x.dtype if x.dtype in _DTYPES else torch.float32)
+        y = _finish(self.matrix.lib, y, self.bias, _out_dtype(x))
         return y if len(lead) == 1 else y.reshape(*lead, self.out_features)
 
     def extra_repr(self):
