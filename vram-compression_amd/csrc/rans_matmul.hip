@@ -1,14 +1,14 @@
 // Decode fused with a matrix product on the matrix cores: out = x * W^T + bias
-// for 16 to 64 rows of x in bf16, W = bf16(code * step) as the decode to a
+// for up to 64 rows of x in bf16, W = bf16(code * step) as the decode to a
 // dense matrix rounds it, sums in f32, on MI355X (gfx950).  The stream format
 // is documented in include/vramc_rans.h, the decode step in rans_device.h.
 //
-// For this many rows the GEMV, whose multiplies are per row of x, is bound by
-// them, and decoding to memory, a dense product and a pass for bias and type
-// spend most of their time outside the decode.  Here each wave decodes its tile 64
-// columns (R symbols) at a time into LDS and the matrix cores multiply
-// behind the decode; the weights never reach memory.  5120x5120 at 32 rows:
-// 37.4 -> 25.9 us.
+// The GEMV's multiplies are per row of x, and beyond 8 or 16 rows bind it;
+// decoding to memory, a dense product and a pass for bias and type spend most
+// of their time outside the decode.  Here each wave decodes its tile 64
+// columns (R symbols) at a time into LDS and the matrix cores multiply behind
+// the decode; the weights never reach memory.  5120x5120 at 32 rows: 37.9 ->
+// 26.2 us a call, 34.0 -> 25.1 in a replayed graph.
 //
 // Bound by the decode's instructions while x is short (5120x5120 at 17 rows
 // 24.5 us, 18 of them what decoding to memory takes) and from there on by the
@@ -16,8 +16,9 @@
 // some 7 TB/s: hence T tile rows to a wave where those reads are many.
 //
 // Shape: a workgroup holds one table copy and rpw groups of T whole tile rows,
-// a wave to each T tiles of a column, up to 16 waves; the waves of a tile row meet in LDS in a fixed
-// order, so no partial sums go through memory and results are deterministic.
+// a wave to each T tiles of a column, up to 16 waves; the waves of a tile row
+// meet in LDS in a fixed order, so no partial sums go through memory and
+// results are deterministic.
 // rpw is the count that puts the fewest waves on the busiest CU.
 #include <hip/hip_runtime.h>
 

@@ -2,9 +2,10 @@
 
 The reference names model integration as its next step (README.md:39) and
 stops at the kernel.  RansLinear is that step: forward(x) runs the fused
-decode+GEMV kernel for decode-sized batches (up to 8 or 16 rows) and, for larger
-batches (prefill), decodes the weight to bf16 once and calls the dense GEMM,
-which is then the faster path.  Inference only: the weight is not a
+decode+GEMV kernel for decode-sized batches (up to 8 or 16 rows), up to 64 rows
+the product on the matrix cores fused with the decode (RansMatrix.matmul, up to
+its matmul_rows), and for larger batches (prefill) decodes the weight to bf16
+once and calls the dense GEMM, each where it is the faster path.  Inference only: the weight is not a
 parameter.
 
 Projections that read the same activations (a decoder layer's q, k, v, or
@@ -25,8 +26,9 @@ from torch.autograd import forward_ad
 
 import rans
 
-# Batches above a matrix's fused_rows_limit decode the weight to bf16 and
-# use the dense GEMM.  The fused GEMV runs up to 8 vectors per launch (4
+# Batches above a matrix's fused_rows_limit multiply with bf16 weights: on the
+# matrix cores behind the decode up to its matmul_rows, beyond them decoded to
+# memory and by the dense GEMM.  The fused GEMV runs up to 8 vectors per launch (4
 # where tiles are taller than 8 rows, the launch splits over column groups,
 # or matrices share a grouped launch), so its time grows with the batch
 # while decode+GEMM stays flat: on MI355X the fused path wins up to 16 rows
