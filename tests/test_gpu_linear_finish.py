@@ -46,3 +46,40 @@ def test_prefill_still_differentiates_and_maps(rans, lib):
         xs = torch.randn(3, 32, 128, generator=g).cuda()
         got = torch.func.vmap(lin)(xs)
         assert torch.allclose(got, torch.stack([lin(v) for v in xs]), rtol=2e-2, atol=0.1)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("bias", [False, True])
+def test_autocast(rans, lib, dtype, bias):
+    """Under autocast the dense product comes in autocast's type, f16 by
+    default; alone and in a group, with more rows than the GEMV takes and than
+    the fused product does.  Bitwise the torch operations on that product."""
+    import rans_linear as L
+    print(f"case autocast {dtype} bias {bias}", flush=True)
+    g = torch.Generator().manual_seed(11)
+    tiling = rans.pick_group_tiling([256, 128], 512)
+    mods = []
+    for rows in (256, 128):
+        codes, step = L.quantize_uniform(torch.randn(rows, 512, generator=g) * 0.05, 3.5)
+        b = torch.randn(rows, generator=g) if bias else None
+        mods.append(L.RansLinear.from_codes(codes, step, b, lib, tiling=(*tiling, 1), tune=False))
+    assert all(m.matrix.fused_rows_limit < 20 <= m.matrix.matmul_rows < 100 for m in mods)
+    ws = [m.matrix.decode() for m in mods]
+    for grouped in (False, True):
+        group = L.LinearGroup(mods) if grouped else None
+        for m in mods:
+            m.group = group
+        for rows in (20, 100):
+            for xt in (torch.float32, torch.bfloat16, torch.float16):
+                x = torch.randn(rows, 512, generator=g).cuda().to(xt)
+                with torch.no_grad(), torch.autocast("cuda", dtype=dtype):
+                    got = [m(x) for m in mods]
+                    if grouped:
+                        y = torch.nn.functional.linear(x.bfloat16(), torch.cat(ws))
+                        ys = y.split([256, 128], dim=1)
+                    else:
+                        ys = [torch.nn.functional.linear(x.bfloat16(), w) for w in ws]
+                for m, y, out in zip(mods, ys, got):
+                    assert y.dtype is dtype and out.dtype is xt
+                    want = y.float() if m.bias is None else y.float() + m.bias
+                    assert torch.equal(out, want.to(xt)), (grouped, rows, xt)

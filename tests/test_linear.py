@@ -24,3 +24,42 @@ def test_ranslinear_fails_without_gpu(rans):
     codes = np.random.default_rng(1).integers(-5, 6, size=(64, 128)).astype(np.int32)
     with pytest.raises(RuntimeError):
         L.RansLinear.from_codes(codes, np.ones(128, np.float32), tune=False)
+
+
+class _Lib:
+    """Stands in for the library: records the calls that would go to the GPU
+    and answers 0, as after a launch."""
+
+    def __init__(self):
+        self.calls = []
+
+    def __getattr__(self, name):
+        return lambda *a: (self.calls.append((name, a)), 0)[1]
+
+
+@pytest.fixture
+def on_cpu(rans, monkeypatch):
+    """rans_linear with CPU tensors taken for plain ones of the GPU."""
+    import rans_linear as L
+    monkeypatch.setattr(L, "_plain", lambda t: True)
+    monkeypatch.setattr(rans, "_stream", lambda: 0)
+    return L
+
+
+@pytest.mark.parametrize("y_dtype", [torch.float32, torch.bfloat16, torch.float16, torch.float64])
+@pytest.mark.parametrize("bias", [False, True])
+def test_finish_takes_the_products_it_has_a_kernel_for(on_cpu, y_dtype, bias):
+    """A product in f16 (what a dense layer returns under autocast's default
+    type) or any other type but f32 and bf16 is finished by torch."""
+    lib = _Lib()
+    y = torch.randn(5, 16, generator=torch.Generator().manual_seed(1)).to(y_dtype)
+    b = torch.full((16,), 0.25) if bias else None
+    for out in (torch.float32, torch.bfloat16, torch.float16):
+        got = on_cpu._finish(lib, y, b, out)
+        assert got.dtype is out and got.shape == y.shape
+        if y_dtype in (torch.float32, torch.bfloat16):
+            assert bool(lib.calls) == (bias or y_dtype is not out)
+        else:
+            assert not lib.calls
+            assert torch.equal(got, (y.float() if b is None else y.float() + b).to(out))
+        lib.calls.clear()

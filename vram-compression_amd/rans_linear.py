@@ -84,14 +84,15 @@ def _plain_bias(bias):
 
 
 def _finish(lib, y, bias, dtype):
-    """(y.float() + bias).to(dtype) for a product y (rows x out_features, f32
-    or bf16, rows possibly wider apart): one pass (rans_linear_finish) where y
-    is a plain tensor, the same torch operations otherwise, bitwise alike."""
+    """(y.float() + bias).to(dtype) for a product y (rows x out_features, rows
+    possibly wider apart): one pass (rans_linear_finish) where y is a plain
+    tensor in f32 or bf16, the same torch operations otherwise (autocast makes
+    products in f16), bitwise alike."""
     if bias is None and y.dtype is dtype and y.is_contiguous():
         return y
     rows, cols = y.shape
-    if (rows and y.stride(1) == 1 and (rows == 1 or y.stride(0) >= cols) and _plain(y)
-            and _plain_bias(bias)):
+    if (rows and y.dtype in (torch.float32, torch.bfloat16) and y.stride(1) == 1
+            and (rows == 1 or y.stride(0) >= cols) and _plain(y) and _plain_bias(bias)):
         out = torch.empty((rows, cols), device=y.device, dtype=dtype)
         rc = lib.rans_linear_finish(y.data_ptr(), _DTYPES[y.dtype], max(y.stride(0), cols),
                                     None if bias is None else bias.data_ptr(), out.data_ptr(),
