@@ -1,5 +1,7 @@
-"""RansLinear host logic (no GPU): the uniform quantiser and the loud
-failure without a device."""
+"""RansLinear host logic (no GPU): the uniform quantiser, the loud
+failure without a device, and what reaches a kernel."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -63,3 +65,44 @@ def test_finish_takes_the_products_it_has_a_kernel_for(on_cpu, y_dtype, bias):
             assert not lib.calls
             assert torch.equal(got, (y.float() if b is None else y.float() + b).to(out))
         lib.calls.clear()
+
+
+class _Matrix:
+    """Stands in for a RansMatrix of 8 rows and 16 columns on the CPU."""
+    rows, cols, fused_rows_limit, matmul_rows = 8, 16, 8, 64
+
+    def __init__(self):
+        self.lib, self.fused = _Lib(), []
+        self.w = torch.randn(8, 16, generator=torch.Generator().manual_seed(4)).bfloat16()
+
+    def decode(self):
+        return self.w
+
+    def matmul(self, x, bias, dtype):
+        self.fused.append(bias)
+        return (x.float() @ self.w.float().t() + (0 if bias is None else bias)).to(dtype)
+
+
+def test_bias_of_another_length_stays_with_torch(on_cpu):
+    """A kernel reads one value per output: a single value, which torch's add
+    broadcasts, and a wrong length, which it refuses, never reach one."""
+    x = torch.randn(20, 16, generator=torch.Generator().manual_seed(5))
+    for rows, kernel in ((20, "fused"), (100, "finish")):
+        m = _Matrix()
+        lin = on_cpu.RansLinear(m)
+        full = torch.linspace(-1, 1, 8)
+        xs = x.repeat(5, 1)[:rows]
+        want = torch.nn.functional.linear(xs.bfloat16(), m.w).float()
+        lin.bias = full
+        lin(xs)
+        assert len(m.fused) == (kernel == "fused")
+        assert len(m.lib.calls) == (kernel == "finish")
+        m.fused.clear(), m.lib.calls.clear()
+        for bias in (full[:1], full[None], torch.tensor(0.5)):
+            lin.bias = bias
+            assert torch.equal(lin(xs), want + bias)
+        for n in (7, 9, 16):
+            lin.bias = torch.zeros(n)
+            with pytest.raises(RuntimeError):
+                lin(xs)
+        assert not m.fused and not m.lib.calls

@@ -77,9 +77,11 @@ def _plain(t):
             and torch._C._len_torch_dispatch_stack() == 0)
 
 
-def _plain_bias(bias):
-    """Whether bias is None or one the kernels read: plain, f32, contiguous."""
-    return bias is None or (_plain(bias) and bias.dtype is torch.float32 and bias.dim() == 1
+def _plain_bias(bias, n):
+    """Whether bias is None or one the kernels read: plain, f32, contiguous,
+    one value for each of n outputs (torch's add broadcasts a single value and
+    refuses other lengths; a kernel would read past the end)."""
+    return bias is None or (_plain(bias) and bias.dtype is torch.float32 and bias.shape == (n,)
                             and bias.is_contiguous())
 
 
@@ -92,7 +94,7 @@ def _finish(lib, y, bias, dtype):
         return y
     rows, cols = y.shape
     if (rows and y.dtype in (torch.float32, torch.bfloat16) and y.stride(1) == 1
-            and (rows == 1 or y.stride(0) >= cols) and _plain(y) and _plain_bias(bias)):
+            and (rows == 1 or y.stride(0) >= cols) and _plain(y) and _plain_bias(bias, cols)):
         out = torch.empty((rows, cols), device=y.device, dtype=dtype)
         rc = lib.rans_linear_finish(y.data_ptr(), _DTYPES[y.dtype], max(y.stride(0), cols),
                                     None if bias is None else bias.data_ptr(), out.data_ptr(),
@@ -203,7 +205,8 @@ class RansLinear(torch.nn.Module):
         if self.group is not None:
             y = self.group.product(self, x, xd.contiguous())
         elif xd.shape[0] > 8 and xd.shape[0] > self.matrix.fused_rows_limit:
-            if (xd.shape[0] <= self.matrix.matmul_rows and _plain(x) and _plain_bias(self.bias)
+            if (xd.shape[0] <= self.matrix.matmul_rows and _plain(x)
+                    and _plain_bias(self.bias, self.out_features)
                     and not torch.is_autocast_enabled("cuda")):
                 y = self.matrix.matmul(xd, self.bias, _out_dtype(x))
                 return y if len(lead) == 1 else y.reshape(*lead, self.out_features)
