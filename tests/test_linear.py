@@ -106,3 +106,36 @@ def test_bias_of_another_length_stays_with_torch(on_cpu):
             with pytest.raises(RuntimeError):
                 lin(xs)
         assert not m.fused and not m.lib.calls
+
+
+class _Device(torch.Tensor):
+    is_cuda = True
+
+
+def test_matmul_checks_its_bias(rans, monkeypatch):
+    """RansMatrix.matmul hands the kernel f32 biases of the matrix's rows
+    only: other types are converted, other lengths and devices refused."""
+    monkeypatch.setattr(rans, "_CUDA", torch.device("cpu"))
+    monkeypatch.setattr(rans, "_stream", lambda: 0)
+    m = object.__new__(rans.RansMatrix)
+    m.rows, m.cols, m.stream_cols, m.lib, m._desc = 8, 64, 64, _Lib(), rans.RansMatrixDesc()
+    seen = []
+
+    def kernel(desc, x, batch, bias, *rest):
+        seen.append(None if bias is None else
+                    np.ctypeslib.as_array((ctypes.c_float * m.rows).from_address(bias)).copy())
+        return 0
+    m.lib.rans_w64_matmul = kernel
+    x = torch.zeros(3, 64).as_subclass(_Device)
+    want = torch.arange(8, dtype=torch.float32)
+    strided = torch.stack([want, -want], 1)[:, 0]
+    for b in (want, want.bfloat16(), want.half(), want.double(), want.int(), strided):
+        m.matmul(x, b)
+        np.testing.assert_array_equal(seen.pop(), want.numpy())
+    m.matmul(x)
+    assert seen.pop() is None
+    for b in (want[:7], want[:1], torch.tensor(1.0), torch.zeros(9), torch.zeros(1, 8),
+              torch.zeros(8, device="meta")):
+        with pytest.raises(ValueError):
+            m.matmul(x, b)
+    assert not seen

@@ -774,8 +774,14 @@ class RansMatrix:
     def matmul(self, x, bias=None, dtype=torch.float32):
         """x @ W^T + bias for up to matmul_rows rows of x, the weights rounded
         to bf16 as decode rounds them and multiplied on the matrix cores with
-        x in bf16, sums in f32 and one rounding to dtype (f32, bf16 or f16)."""
+        x in bf16, sums in f32 and one rounding to dtype (f32, bf16 or f16).
+        bias: one value for each row of W, on x's device; used as f32."""
         assert x.is_cuda and x.dim() == 2 and x.shape[1] == self.cols
+        if bias is not None:  # the kernel reads rows f32 values behind a pointer
+            if bias.device != x.device or bias.shape != (self.rows,):
+                raise ValueError(f"bias must have {self.rows} values on {x.device}, got "
+                                 f"{tuple(bias.shape)} on {bias.device}")
+            bias = bias.float().contiguous()
         x, _ = _x_operand(x.to(torch.bfloat16), self.stream_cols)
         if x.data_ptr() % 16:  # the kernel reads 16 bytes at a time
             x = x.clone()
