@@ -139,3 +139,41 @@ def test_matmul_checks_its_bias(rans, monkeypatch):
         with pytest.raises(ValueError):
             m.matmul(x, b)
     assert not seen
+
+
+def test_what_watches_a_tensor_keeps_it_from_the_kernels(rans, monkeypatch):
+    """A kernel called through a pointer is hidden from gradients, forward
+    mode, vmap and dispatch and function modes, so tensors that one of these
+    watches are not plain; the mode of a default device watches nothing."""
+    import rans_linear as L
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True)
+    monkeypatch.setattr(rans, "_device", lambda: -1)
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    t = torch.zeros(3)
+    assert L._plain(t)
+    for mode in (Function, Dispatch):
+        with mode():
+            assert not L._plain(t)
+    with torch.device("cpu"):
+        assert L._plain(t)
+        with Function():
+            assert not L._plain(t)
+    with forward_ad.dual_level():
+        assert not L._plain(t)
+    seen = []
+    torch.func.vmap(lambda v: (seen.append(L._plain(v)), v)[1])(torch.zeros(2, 3))
+    assert seen == [False]
+    assert not L._plain(torch.zeros(3, requires_grad=True))
+    assert not L._plain(torch.nn.Parameter(t, requires_grad=False))
+    assert L._plain(t)

@@ -23,6 +23,7 @@ import weakref
 import numpy as np
 import torch
 from torch.autograd import forward_ad
+from torch.utils._device import DeviceContext
 
 import rans
 
@@ -66,15 +67,22 @@ _peek_functorch = getattr(getattr(torch._C, "_functorch", None), "peek_interpret
                           lambda: None)
 
 
+def _function_mode():
+    """Whether a torch function mode other than a default device is active."""
+    n = torch._C._len_torch_function_stack()
+    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
+                         for i in range(n))
+
+
 def _plain(t):
     """Whether t is an ordinary tensor of the current GPU that nothing else
-    watches: no gradient, forward-mode, vmap, tracing or dispatch mode that an
-    operation outside torch would be hidden from."""
+    watches: no gradient, forward-mode, vmap, tracing, dispatch or function
+    mode that an operation outside torch would be hidden from."""
     return (type(t) is torch.Tensor and t.is_cuda and not t.requires_grad
             and t.get_device() == rans._device() and not torch.compiler.is_compiling()
             and forward_ad._current_level < 0 and _peek_functorch() is None
             and torch._C._get_tracing_state() is None
-            and torch._C._len_torch_dispatch_stack() == 0)
+            and torch._C._len_torch_dispatch_stack() == 0 and not _function_mode())
 
 
 def _plain_bias(bias, n):
