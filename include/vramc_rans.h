@@ -216,6 +216,11 @@ int rans_w64_matmul(const rans_w64_matrix* m, const void* x, int batch, const fl
                     void* out, int out_dtype, hipStream_t stream);
 int rans_matmul_rows(const rans_w64_matrix* m);
 
+/* Tile rows that a wave of rans_w64_matmul takes for this matrix and batch on
+ * an MI355X, 0 where it takes neither (host code, no GPU needed).  Results are
+ * the same for any.  No reference counterpart. */
+int rans_matmul_tiles(const rans_w64_matrix* m, int batch);
+
 /* Decode to a dense bf16 matrix out[r,c] = bf16(code[r,c]*step[c]) (round to
  * nearest even).  Replaces launch_rans_decode (rans_gemv.cu:155-162). */
 int rans_w64_decode(const rans_w64_matrix* m, void* out_bf16, hipStream_t stream);

@@ -182,3 +182,30 @@ def test_fused_rows_limit_follows_the_planner(rans, lib):
     assert rans.fused_rows_limit(two, lib) == 8
     bad = _desc(rans, mtw=70000)                # outside the format: no launch at all
     assert rans.fused_rows_limit(bad, lib) == 8
+
+
+@pytest.mark.parametrize("rows,cols,R,C,esc,batch,tiles", [
+    # the faster one where the two measured 10% and more apart
+    (5120, 5120, 8, 1024, False, 32, 2), (5120, 5120, 8, 1024, True, 17, 1),
+    (6400, 5120, 8, 1024, False, 17, 2), (6400, 5120, 8, 1024, True, 17, 2),
+    (4096, 4096, 8, 1024, True, 24, 1), (4096, 4096, 8, 1024, True, 64, 2),
+    (1536, 8960, 3, 2240, False, 32, 4), (1536, 8960, 3, 2240, True, 17, 1),
+    (2048, 8192, 4, 2048, True, 24, 1), (2048, 8192, 4, 2048, True, 64, 4),
+    (25600, 1024, 16, 256, True, 24, 2), (10240, 3200, 16, 640, False, 24, 1),
+    (8192, 2048, 16, 512, True, 48, 1), (1536, 17920, 3, 2240, True, 24, 4),
+    # one tile row of 35 fills the wave; two of these do not fit the LDS
+    (8960, 1536, 35, 192, False, 64, 1), (2064, 8704, 16, 1088, False, 64, 1),
+    # no kernel for these tiles, or for so many rows
+    (2560, 9728, 2, 2432, False, 32, 0), (5120, 5120, 8, 1024, False, 65, 0),
+])
+def test_matmul_tiles(rans, lib, rows, cols, R, C, esc, batch, tiles):
+    d = _desc(rans, rows=rows, cols=cols, R=R, C=C, mtw=int(R * C * 3.3 / 16))
+    d.flags = 0 if esc else rans.F_NO_ESCAPES
+    assert lib.rans_matmul_tiles(ctypes.byref(d), batch) == tiles
+
+
+def test_matmul_tiles_refuses(rans, lib):
+    d = _desc(rans)
+    assert lib.rans_matmul_tiles(None, 8) == -2
+    assert lib.rans_matmul_tiles(ctypes.byref(_desc(rans, cols=4000)), 8) == -2
+    assert lib.rans_matmul_tiles(ctypes.byref(d), 0) == -4

@@ -2,6 +2,8 @@
 x, steps that are powers of two) against the decoded matrix in 64 bits, over
 the tile heights, one and several tile rows to a wave, ragged ends of both, and
 the calls that RansLinear keeps on the dense product."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -21,8 +23,8 @@ def _matrix(rans, lib, rows, cols, R, C, esc, seed):
     return rans.RansMatrix(rans.encode(codes, R, C, 1), torch.from_numpy(step), lib)
 
 
-# the wide ones read 136 MB or more of x at 64 rows: several tile rows to a
-# wave, an odd number in all, which 2 and 4 leave over
+# the wide ones read 136 MB or more of x at 64 rows, an odd number of tile
+# rows most of them
 WIDE = [(513, 6528, 3, 1088), (516, 8704, 4, 1088), (1032, 8704, 8, 1088), (4368, 4096, 16, 512),
         (2064, 8704, 16, 1088)]  # of the last, two tile rows to a wave do not fit the LDS
 
@@ -43,6 +45,29 @@ def test_exact_sums(rans, lib, rows, cols, R, C, esc):
         assert torch.equal(m.matmul(x), want), nb
         assert torch.equal(m.matmul(x.float(), bias, torch.bfloat16), (want + bias).bfloat16()), nb
         assert torch.equal(m.matmul(x, bias, torch.float16), (want + bias).half()), nb
+
+
+# many short tiles: several tile rows to a wave from these rows of x on,
+# an odd number of tile rows, which 2 and 4 leave over
+@pytest.mark.parametrize("rows,cols,R,C,tiles", [
+    (2895, 256, 3, 64, 4), (3876, 320, 4, 64, 4), (8968, 192, 8, 64, 2), (5672, 768, 8, 192, 2),
+    (8976, 1024, 16, 256, 2)])
+@pytest.mark.parametrize("esc", [0.0, 0.02])
+def test_several_tile_rows(rans, lib, rows, cols, R, C, tiles, esc):
+    m = _matrix(rans, lib, rows, cols, R, C, esc, rows + cols)
+    w = m.decode().double()
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    bias = torch.randn(rows, device="cuda", generator=g)
+    taken = []
+    for nb in (1, 17, 33, 48, 64):
+        taken.append(lib.rans_matmul_tiles(ctypes.byref(m._desc), nb))
+        print(f"case matmul {rows}x{cols} R={R} C={C} esc={esc} rows of x {nb} T={taken[-1]}",
+              flush=True)
+        x = torch.randint(-4, 5, (nb, cols), device="cuda", generator=g).bfloat16()
+        want = (x.double() @ w.t()).float()
+        assert torch.equal(m.matmul(x), want), nb
+        assert torch.equal(m.matmul(x, bias, torch.bfloat16), (want + bias).bfloat16()), nb
+    assert taken[0] == 1 and taken[-1] == tiles
 
 
 def test_refuses(rans, lib):

@@ -32,6 +32,7 @@ namespace {
 
 constexpr int kMmMaxWaves = 16;
 constexpr int kMmMaxRows = 64;
+constexpr int kMmCus = 256;  // of an MI355X, for the questions asked without a device
 constexpr int kMmStaticLds = (int)sizeof(TabEntry<false>) * (int)kProbM;
 // Row stride of a wave's R x 64 weights in LDS: 16 bytes beyond the 128, so
 // that 16 rows read as 16-byte fragments spread over the banks.
@@ -275,14 +276,30 @@ __global__ void __launch_bounds__(64 * kMmMaxWaves) rans_w64_matmul_kernel(Matmu
 
 // Tile rows a wave can take at once: as many as fill the matrix cores' 16
 // rows, and two of 16.  Every wave reads its columns of x for itself, so with
-// T of them x is read T times less; in exchange the launch has T times fewer
-// waves.  Taken where one tile row at a time would read 136 MB of x or more
-// from the caches, some 20 us (one and T, us: 5120x5120 in 8-row tiles, 32
-// rows, 168 MB, 34.1 and 25.9; 6400x5120, 17 rows, 139 MB, 34.2 and 28.8;
-// 4096x4096, 32 rows, 134 MB, 19.4 and 22.3; 12800x2048 in 16-row tiles, 17
-// rows, 56 MB, 20.5 and 22.8, 48 rows, 157 MB, 32.4 and 25.6).
+// T of them x is read T times less; in exchange T times fewer waves each
+// decode T times the symbols, one tile's after the other's.
 constexpr int mm_tiles(int R) { return R <= 4 ? 4 : R <= 16 ? 2 : 1; }
-constexpr int64_t kMmWideReads = 136 << 20;
+
+// What T decides of a launch's time, in ps: a wave decodes a symbol in 50 ns
+// alone on its SIMD and in 14 for every wave the SIMD holds, and escapes cost
+// three symbols a column step and tile; x comes from the caches at 9 TB/s; a
+// column step of a 16x16 block of the product takes its SIMD 40 ns.  Of 45
+// matrices at 17 to 64 rows the better T by this is within 0.3% of the faster
+// one on average and within 12% at worst (a limit on the bytes of x was 3.6%
+// and 61% off).  One and T tile rows, us from a replayed graph: 5120x5120 in
+// 8-row tiles, 32 rows, 34.8 and 26.5; 6400x5120, 17 rows, 31.6 and 23.9;
+// 25600x1024 in 16-row tiles, 24 rows, 27.4 and 22.5; 4096x4096 in 8-row
+// tiles, 24 rows, 17.7 and 21.6; 10240x3200 in 16-row tiles, 24 rows, 22.3 and
+// 29.0; 1536x8960 in 3-row tiles, 32 rows, 35.5 and 26.2, with escapes 36.2
+// and 35.8; 2048x8192 in 4-row tiles with escapes, 17 rows, 23.5 and 37.9.
+int64_t matmul_cost(const rans_w64_matrix* m, int nb, int T, int cus) {
+    const int64_t nrb = m->rows / m->R, steps = m->C / 64, simds = 4 * cus;
+    const int64_t waves = (nrb + T - 1) / T * (m->cols / m->C);
+    const int64_t symbols = steps * (m->R + (m->flags & RANS_F_NO_ESCAPES ? 0 : 3));
+    const int64_t blocks = waves * steps * ((T * m->R + 15) / 16) * ((nb + 15) / 16);
+    return symbols * T * std::max<int64_t>(50000, 14000 * waves / simds) +
+           nrb * nb * m->cols * 2 / T / 9 + 40000 * blocks / simds;
+}
 
 // Groups of T tile rows per workgroup: of the counts that put the fewest
 // waves on the busiest CU when the workgroups spread evenly the largest
@@ -308,21 +325,27 @@ struct MatmulShape {
 };
 
 MatmulShape matmul_shape(const rans_w64_matrix* m, int nb, int cus) {
-    if ((int64_t)(m->rows / m->R) * nb * m->cols * 2 >= kMmWideReads)
-        if (const int rpw = matmul_rpw(m, mm_tiles(m->R), cus)) return {mm_tiles(m->R), rpw};
+    const int T = mm_tiles(m->R);
+    if (T > 1 && matmul_cost(m, nb, T, cus) < matmul_cost(m, nb, 1, cus))
+        if (const int rpw = matmul_rpw(m, T, cus)) return {T, rpw};
     return {1, matmul_rpw(m, 1, cus)};
 }
 
-// The rows up to which this is the faster path: twice the rows a wave takes
+// The rows up to which this path is taken: twice the rows a wave takes
 // (some 4 bytes of x read per weight, what writing and reading the weight
 // takes), in whole blocks of 16, or all 64 for matrices of up to 4M weights,
-// whose time is in the launches.  Against decoding and the dense product (us,
-// from a replayed graph, without the host's part): 5120x5120 at 32 rows 25.1
-// to 34.0, at 48 37.9 to 40.0, at 64 45.7 to 37.2; 1536x1536 at 64 11.5 to
-// 16.6; 12800x2048 in 16-row tiles at 64 27.8 to 33.0; 8960x1536 in 35-row
-// tiles at 64 17.8 to 27.6; 1536x8960 in 3-row tiles at 32 25.9 to 33.5, at 64
-// 37.4 to 36.2.  Shorter tiles than 3 rows stay on the dense product
-// (2560x9728 in 2-row tiles at 32 rows 39.1 to 37.5).
+// whose time is in the launches.  Against decoding, the dense product and the
+// last pass (us, from a replayed graph over three copies, without the host's
+// part, which is 37 us for those three): 5120x5120 at 32 rows 26.5 to 34.2, at
+// 64 47.2 to 38.2; 1536x1536 at 64 11.4 to 16.4; 12800x2048 in 16-row tiles at
+// 64 27.7 to 33.6; 8960x1536 in 35-row tiles at 64 18.4 to 27.8; 1536x8960 in
+// 3-row tiles at 32 26.2 to 34.3.  Of 45 matrices it is behind at its limit
+// for five: by 5% for 1536x8960 with escapes at 32 (36.2 to 34.3), 6% for
+// 2048x8192 in 4-row tiles with escapes (34.0 to 31.9), 5% for 9600x3200 at 64
+// (38.8 to 36.8), 1% for the others.  Where x is short beside the weight the
+// line is on the safe side: 4096x4096 at 48 rows would take 20.6 (29.3),
+// 1536x17920 54.4 (74.4), 5120x5120 39.2 (40.4).  Shorter tiles than 3 rows
+// stay on the dense product (2560x9728 in 2-row tiles at 32 rows 39.1 to 37.5).
 int matmul_max_rows(const rans_w64_matrix* m, int cus) {
     if (!matmul_rpw(m, 1, cus)) return 0;
     if ((int64_t)m->rows * m->cols <= (4 << 20)) return kMmMaxRows;
@@ -369,7 +392,15 @@ int launch_matmul(const MatmulArgs& a, int T, hipStream_t stream) {
 extern "C" int rans_matmul_rows(const rans_w64_matrix* m) {
     if (!valid_geometry(m)) return RANS_EGEOMETRY;
     if (!matmul_compiled(m) || (int64_t)kMmMaxRows * m->cols * 2 > INT32_MAX) return 0;
-    return matmul_max_rows(m, 256);
+    return matmul_max_rows(m, kMmCus);
+}
+
+extern "C" int rans_matmul_tiles(const rans_w64_matrix* m, int batch) {
+    if (!valid_geometry(m)) return RANS_EGEOMETRY;
+    if (batch <= 0) return RANS_EARG;
+    if (!matmul_compiled(m) || batch > kMmMaxRows || (int64_t)batch * m->cols * 2 > INT32_MAX) return 0;
+    const MatmulShape shape = matmul_shape(m, batch, kMmCus);
+    return shape.rpw ? shape.T : 0;
 }
 
 extern "C" int rans_w64_matmul(const rans_w64_matrix* m, const void* x, int batch, const float* bias,

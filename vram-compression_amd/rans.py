@@ -79,7 +79,8 @@ EXPORTS = ("rans_w64_gemv", "rans_w64_gemv_noalloc", "rans_gemv_workspace_bytes"
            "rans_gemv_rows2", "rans_w64_gemv_group", "launch_rans_gemv", "launch_rans_decode",
            "rans_w64_decode",
            "rans_w64_decode_codes", "rans_linear_finish",
-           "rans_w64_matmul", "rans_matmul_rows", "launch_int4_gemv", "bf16_gemv", "rans_build_table",
+           "rans_w64_matmul", "rans_matmul_rows", "rans_matmul_tiles",
+           "launch_int4_gemv", "bf16_gemv", "rans_build_table",
            "rans_table_lds",
            "rans_table_lds4",
            "rans_w64_encode", "rans_w64_encode_fetch", "rans_w64_encode_counts",
@@ -136,6 +137,7 @@ def load_lib(path=LIB):
                                ctypes.c_int),
         "rans_w64_matmul": ([D, P, ctypes.c_int, P, P, ctypes.c_int, P], ctypes.c_int),
         "rans_matmul_rows": ([D], ctypes.c_int),
+        "rans_matmul_tiles": ([D, ctypes.c_int], ctypes.c_int),
         "launch_int4_gemv": ([P, P, P, ctypes.c_int, ctypes.c_int, P], ctypes.c_int),
         "bf16_gemv": ([P, P, P, ctypes.c_int, ctypes.c_int, P], ctypes.c_int),
         "rans_build_table": ([P, I64, P, P, P], ctypes.c_int),
