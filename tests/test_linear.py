@@ -43,7 +43,7 @@ class _Lib:
 def on_cpu(rans, monkeypatch):
     """rans_linear with CPU tensors taken for plain ones of the GPU."""
     import rans_linear as L
-    monkeypatch.setattr(L, "_plain", lambda t: True)
+    monkeypatch.setattr(L, "_plain", lambda *t: True)
     monkeypatch.setattr(rans, "_stream", lambda: 0)
     return L
 
@@ -161,7 +161,7 @@ def test_what_watches_a_tensor_keeps_it_from_the_kernels(rans, monkeypatch):
             return func(*args, **(kwargs or {}))
 
     t = torch.zeros(3)
-    assert L._plain(t)
+    assert L._plain(t) and L._plain(t, None) and L._plain(t, t)
     for mode in (Function, Dispatch):
         with mode():
             assert not L._plain(t)
@@ -174,6 +174,6 @@ def test_what_watches_a_tensor_keeps_it_from_the_kernels(rans, monkeypatch):
     seen = []
     torch.func.vmap(lambda v: (seen.append(L._plain(v)), v)[1])(torch.zeros(2, 3))
     assert seen == [False]
-    assert not L._plain(torch.zeros(3, requires_grad=True))
-    assert not L._plain(torch.nn.Parameter(t, requires_grad=False))
+    for other in (torch.zeros(3, requires_grad=True), torch.nn.Parameter(t, requires_grad=False)):
+        assert not L._plain(other) and not L._plain(t, other) and not L._plain(other, t)
     assert L._plain(t)

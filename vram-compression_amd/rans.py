@@ -783,7 +783,8 @@ class RansMatrix:
             if bias.device != x.device or bias.shape != (self.rows,):
                 raise ValueError(f"bias must have {self.rows} values on {x.device}, got "
                                  f"{tuple(bias.shape)} on {bias.device}")
-            bias = bias.float().contiguous()
+            if bias.dtype is not torch.float32 or not bias.is_contiguous():
+                bias = bias.float().contiguous()
         x, _ = _x_operand(x.to(torch.bfloat16), self.stream_cols)
         if x.data_ptr() % 16:  # the kernel reads 16 bytes at a time
             x = x.clone()

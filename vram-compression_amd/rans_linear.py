@@ -67,29 +67,35 @@ _peek_functorch = getattr(getattr(torch._C, "_functorch", None), "peek_interpret
                           lambda: None)
 
 
-def _function_mode():
-    """Whether a torch function mode other than a default device is active."""
-    n = torch._C._len_torch_function_stack()
-    return n > 0 and any(type(torch._C._get_function_stack_at(i)) is not DeviceContext
-                         for i in range(n))
+def _function_mode(n):
+    """Whether one of n torch function modes is not just a default device."""
+    return any(type(torch._C._get_function_stack_at(i)) is not DeviceContext for i in range(n))
 
 
-def _plain(t):
-    """Whether t is an ordinary tensor of the current GPU that nothing else
-    watches: no gradient, forward-mode, vmap, tracing, dispatch or function
-    mode that an operation outside torch would be hidden from."""
-    return (type(t) is torch.Tensor and t.is_cuda and not t.requires_grad
-            and t.get_device() == rans._device() and not torch.compiler.is_compiling()
-            and forward_ad._current_level < 0 and _peek_functorch() is None
-            and torch._C._get_tracing_state() is None
-            and torch._C._len_torch_dispatch_stack() == 0 and not _function_mode())
+def _plain(*tensors):
+    """Whether the tensors (or None) are ordinary ones of the current GPU that
+    nothing else watches: no gradient, forward-mode, vmap, tracing, dispatch or
+    function mode that an operation outside torch would be hidden from."""
+    if (torch.compiler.is_compiling() or forward_ad._current_level >= 0
+            or _peek_functorch() is not None or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() > 0):
+        return False
+    modes = torch._C._len_torch_function_stack()
+    if modes and _function_mode(modes):
+        return False
+    device = rans._device()
+    for t in tensors:
+        if t is not None and not (type(t) is torch.Tensor and t.is_cuda and not t.requires_grad
+                                  and t.get_device() == device):
+            return False
+    return True
 
 
-def _plain_bias(bias, n):
-    """Whether bias is None or one the kernels read: plain, f32, contiguous,
+def _takes_bias(bias, n):
+    """Whether bias is None or laid out as the kernels read it: f32, contiguous,
     one value for each of n outputs (torch's add broadcasts a single value and
     refuses other lengths; a kernel would read past the end)."""
-    return bias is None or (_plain(bias) and bias.dtype is torch.float32 and bias.shape == (n,)
+    return bias is None or (bias.dtype is torch.float32 and bias.shape == (n,)
                             and bias.is_contiguous())
 
 
@@ -102,7 +108,8 @@ def _finish(lib, y, bias, dtype):
         return y
     rows, cols = y.shape
     if (rows and y.dtype in (torch.float32, torch.bfloat16) and y.stride(1) == 1
-            and (rows == 1 or y.stride(0) >= cols) and _plain(y) and _plain_bias(bias, cols)):
+            and (rows == 1 or y.stride(0) >= cols) and _takes_bias(bias, cols)
+            and _plain(y, bias)):
         out = torch.empty((rows, cols), device=y.device, dtype=dtype)
         rc = lib.rans_linear_finish(y.data_ptr(), _DTYPES[y.dtype], max(y.stride(0), cols),
                                     None if bias is None else bias.data_ptr(), out.data_ptr(),
@@ -137,8 +144,8 @@ class LinearGroup:
 
     def product(self, member, x, xd):
         """member's x @ W^T (no bias) for the module input x, flattened and
-        converted to xd (rows x in_features, f32 or bf16); f32, or bf16 from
-        the dense GEMM."""
+        converted to xd (rows x in_features, f32 or bf16); f32, or as the
+        dense GEMM makes it (bf16, or autocast's type)."""
         i = next(j for j, m in enumerate(self.members) if m is member)
         if (self._x is not None and self._x() is x and self._version == x._version
                 and i in self._pending):
@@ -213,8 +220,8 @@ class RansLinear(torch.nn.Module):
         if self.group is not None:
             y = self.group.product(self, x, xd.contiguous())
         elif xd.shape[0] > 8 and xd.shape[0] > self.matrix.fused_rows_limit:
-            if (xd.shape[0] <= self.matrix.matmul_rows and _plain(x)
-                    and _plain_bias(self.bias, self.out_features)
+            if (xd.shape[0] <= self.matrix.matmul_rows and _plain(x, self.bias)
+                    and _takes_bias(self.bias, self.out_features)
                     and not torch.is_autocast_enabled("cuda")):
                 y = self.matrix.matmul(xd, self.bias, _out_dtype(x))
                 return y if len(lead) == 1 else y.reshape(*lead, self.out_features)
