@@ -39,3 +39,38 @@ def test_decode_launches(rans, lib, rows, cols, R, C, S):
         rest = torch.cat([buf[:shift], buf[shift + n:]])
         assert bool((rest == 7.0).all()), "stored outside the output"
     np.testing.assert_array_equal(m.decode_codes().cpu().numpy(), codes)
+
+
+@pytest.mark.parametrize("rows,cols,R,C,S", [
+    (16386, 4096, 2, 2048, 1), (8196, 8192, 4, 1024, 2), (10928, 6144, 8, 1536, 4),
+    (16400, 4096, 16, 512, 2), (13120, 5120, 20, 640, 1),
+    (15424, 4352, 16, 1088, 1),   # 3856 tiles: one round, no wave takes a second
+    (29155, 2304, 35, 576, 1),    # the same, odd tile height
+    (1048580, 64, 1, 64, 1)])     # single rows: nothing to pair
+def test_paired_rows(rans, lib, rows, cols, R, C, S):
+    """Outputs of 64M weights and more, whose rows are stored in pairs, over
+    tile heights, states per lane and both launches: every value, escapes in
+    either row of a pair, in both, and in the row that an odd height leaves
+    over; at a 4-byte boundary and 2 bytes past one, where rows go out singly."""
+    print(f"case paired decode {rows}x{cols} R={R} C={C} S={S}", flush=True)
+    assert rows * cols >= 64 << 20
+    rng = np.random.default_rng(rows + cols)
+    few = 2 * R  # rows of codes, repeated over the height
+    codes = np.rint(rng.laplace(size=(few, cols)) * 2).astype(np.int32)
+    hit = rng.random(codes.shape) < 0.003
+    codes[hit] = rng.integers(128, 900, int(hit.sum()))
+    codes[0, ::31] = -300                # the first row of a pair,
+    codes[min(1, few - 1), ::17] = 301   # the second, and both
+    codes[R - 1, -3:] = 302              # the last row of a tile, the last columns
+    codes = np.resize(codes, (rows, cols))
+    step = (rng.random(cols) + 0.25).astype(np.float32)
+    m = rans.RansMatrix(rans.encode(codes, R, C, S), torch.from_numpy(step), lib)
+    dev = torch.from_numpy(codes).cuda()
+    want = (dev.float() * torch.from_numpy(step).cuda()).bfloat16()
+    n = rows * cols
+    for shift in (0, 1):  # of the output, in elements
+        buf = torch.full((n + 8,), 7.0, device="cuda", dtype=torch.bfloat16)
+        assert torch.equal(m.decode(buf[shift:shift + n].view(rows, cols)), want), shift
+        rest = torch.cat([buf[:shift], buf[shift + n:]])
+        assert bool((rest == 7.0).all()), "stored outside the output"
+    assert torch.equal(m.decode_codes(), dev)

@@ -34,7 +34,8 @@ def test_ranslinear_matches_dense(rans, lib):
             ref = torch.nn.functional.linear(x.double(), wd) + b.double()
             assert y.dtype == dt and tuple(y.shape) == tuple(ref.shape)
             assert _rel(y, ref) <= tol[dt], (shape, dt, _rel(y, ref))
-    # prefill-sized batch: bf16 decode + dense GEMM
+    # more rows than the GEMV takes: the fused product of bf16 weights
+    assert lin.matrix.matmul_rows == 64
     x = torch.randn(32, 1536, generator=g)
     y = lin(x.cuda())
     ref = torch.nn.functional.linear(x.double(), wd) + b.double()
@@ -70,8 +71,9 @@ def test_tiny_qwen2_with_rans_linears(rans, lib):
         a = dense(ids).logits
         b = coded(ids).logits
         assert _rel(b, a) <= 1e-3
-        # a longer prompt (more rows than any matrix's fused_rows_limit) takes
-        # the prefill path (bf16-decoded weights + dense GEMM)
+        # a longer prompt (more rows than any matrix's fused_rows_limit)
+        # multiplies bf16 weights: the groups decode and run a dense GEMM,
+        # o_proj and down_proj the fused product
         long_ids = torch.randint(0, 512, (1, 20), generator=torch.Generator().manual_seed(2)).cuda()
         assert _rel(coded(long_ids).logits, dense(long_ids).logits) <= 2e-2
         # one decode step: two grouped launches per layer (q/k/v, gate/up)
@@ -174,7 +176,7 @@ def test_linear_group_prefill_one_gemm(rans, lib):
 
 def test_linears_with_odd_multiple_of_32_inputs(rans, lib):
     """in_features an odd multiple of 32 (96, 1568): RansLinear (GEMV and
-    prefill paths) and a grouped pair built by replace_linears match their
+    fused product) and a grouped pair built by replace_linears match their
     dense twins; the matrices are stored with 32 appended columns."""
     import rans_linear as L
     print("case RansLinear odd-32 in_features", flush=True)
@@ -216,3 +218,45 @@ def test_linears_with_odd_multiple_of_32_inputs(rans, lib):
     xd = x.double()
     ref = (xd @ wq["gate_proj"].T) * (xd @ wq["up_proj"].T)
     assert _rel(y, ref) <= 2e-3
+
+
+@pytest.mark.parametrize("in_f", [512, 1568])  # the second with 32 appended columns
+@pytest.mark.parametrize("bias", [False, True])
+def test_dense_route(rans, lib, in_f, bias):
+    """More rows than the fused product takes, alone and in a group: decode,
+    the dense GEMM and the finishing pass, bitwise the torch operations on the
+    decoded weight, and no further from 64 bits than two roundings to bf16 (of
+    weights and product) and one to the output type: 3 * 2^-9 of each term, on
+    average far less."""
+    import rans_linear as L
+    print(f"case RansLinear dense route {in_f} bias {bias}", flush=True)
+    g = torch.Generator().manual_seed(in_f)
+    tiling = rans.pick_group_tiling([264, 128], in_f)
+    mods, wds = [], []
+    for rows in (264, 128):
+        codes, step = L.quantize_uniform(torch.randn(rows, in_f, generator=g) * 0.05, 3.5)
+        codes[3, 5], codes[-1, -1] = 300, -301  # escapes
+        b = torch.randn(rows, generator=g) if bias else None
+        mods.append(L.RansLinear.from_codes(codes, step, b, lib, tiling=(*tiling, 1), tune=False))
+        wds.append(torch.from_numpy(codes).double() * torch.from_numpy(step).double())
+    assert all(m.matrix.matmul_rows <= 64 for m in mods)
+    ws = [m.matrix.decode() for m in mods]
+    for rows in (65, 100, 512):
+        for dt in (torch.float32, torch.bfloat16, torch.float16):
+            x = torch.randn(rows, in_f, generator=g).cuda().to(dt)
+            alone = [m(x) for m in mods]
+            group = L.LinearGroup(mods)
+            for m in mods:
+                m.group = group
+            grouped = [m(x) for m in mods]
+            for m in mods:
+                m.group = None
+            xb = x.bfloat16()
+            both = torch.nn.functional.linear(xb, torch.cat(ws)).split([264, 128], dim=1)
+            for m, w, wd, y, a, ys in zip(mods, ws, wds, both, alone, grouped):
+                for got, prod in ((a, torch.nn.functional.linear(xb, w)), (ys, y)):
+                    want = prod.float() if m.bias is None else prod.float() + m.bias
+                    assert got.dtype is dt and torch.equal(got, want.to(dt)), (rows, dt)
+                    ref = xb.double().cpu() @ wd.t()
+                    ref = ref if m.bias is None else ref + m.bias.double().cpu()
+                    assert _rel(got, ref) <= 3 * 2 ** -9, (rows, dt)
