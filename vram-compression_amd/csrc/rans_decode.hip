@@ -105,6 +105,9 @@ __global__ void __launch_bounds__(64 * kMaxDecodeWaves) rans_w64_decode_kernel(D
         const int tc = min(tile, a.ntiles - 1);
         h.to = load_tile_off(a.tile_off, tc);
         h.tp = a.esc_tileptr[tc + min(lane, 1)];
+        // keep these loads first: the block's copy waits for the extent, and
+        // left alone the compiler takes its end after all the others
+        asm volatile("" ::: "memory");
         h.tmv = a.tile_meta[tc];
 #pragma unroll
         for (int s = 0; s < S; s++) h.len[s] = a.slen[tc * nst + 64 * s + lane];
