@@ -10,7 +10,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("rows,cols,R,C,S", [
-    (2050, 256, 1, 64, 1),      # 8200 tiles: several per wave, single rows
+    (2050, 256, 1, 64, 1),      # 8200 tiles: two workgroups a CU, single rows
+    (9001, 256, 1, 64, 1),      # 36004: five rounds of them, the last one partial
     (4100, 2048, 2, 256, 1),    # 16400 tiles
     (4098, 2112, 3, 192, 1),    # odd tile height, three column steps per tile
     (8960, 960, 35, 192, 1),    # one round, odd tile height

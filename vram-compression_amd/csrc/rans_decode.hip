@@ -67,11 +67,11 @@ __device__ __forceinline__ uint32_t quad_swap(uint32_t v) {
 // 30.9 us, 8960x1536 and 512 rows 35.5 against 32.6; at 13824x5120, 141 MB,
 // and 64 rows 74.2 against 79.4).
 //
-// LOOP: workgroups stay, one per CU; each wave takes tiles first, first +
+// LOOP: workgroups stay, one or two a CU; each wave takes tiles first, first +
 // stride, ... and copies the next tile's block as soon as it has decoded the
-// last, so the table is copied once per CU and a wave waits for no other.
-// 5120x5120 in 8x1024 tiles (3200 of them, formerly in workgroups of one
-// wave, 4 waves on a CU) 37.7 -> 19 us.
+// last, so the table is copied once per workgroup and a wave waits for no
+// other.  5120x5120 in 8x1024 tiles (3200 of them, formerly in workgroups of
+// one wave, 4 waves on a CU) 37.7 -> 17.6 us.
 template <int R, int S, int MODE, bool PAIR, bool LOOP>
 __global__ void __launch_bounds__(64 * kMaxDecodeWaves) rans_w64_decode_kernel(DecodeArgs a) {
     __shared__ __align__(16) TabEntry<false> tab[kProbM];
@@ -150,11 +150,10 @@ __global__ void __launch_bounds__(64 * kMaxDecodeWaves) rans_w64_decode_kernel(D
 #pragma unroll
         for (int s = 0; s < S; s++) st0[s] = initial_state(raw, bit0[s], cur.len[s]);
         init_lanes(L, tab, raw, st0, off0);
-        // One block of NU <= KU column steps, i.e. NG column groups of 64.  The
-        // loop below runs whole blocks only (no early exit): exits after 1, 2
-        // or 3 steps' stores would meet at the loop latch, and the compiler
-        // would then wait there for the stores of the longest path.  A partial
-        // last block follows it.
+        // One block of NU <= KU column steps.  The loop below runs whole blocks
+        // only (no early exit): exits after 1, 2 or 3 steps' stores would meet
+        // at the loop latch, and the compiler would then wait there for the
+        // stores of the longest path.  A partial last block follows it.
         auto run_block = [&](int k0, auto nu_) {
             constexpr int NU = decltype(nu_)::value;
             float sv[KU][S];
@@ -260,28 +259,55 @@ __global__ void __launch_bounds__(64 * kMaxDecodeWaves) rans_w64_decode_kernel(D
     }
 }
 
-// Waves per decode workgroup when one workgroup per CU takes all the tiles
-// (loop): as many as the LDS holds, but no more than give every wave the same
-// number of tiles.  Otherwise (int32 codes, whose time is their writes), of
-// the counts that put the fewest waves on the busiest CU when the workgroups
-// spread evenly the largest, from 4 up: workgroups of fewer waves fill the
-// LDS with tables.
-int decode_waves(const rans_w64_matrix* m, int64_t ntiles, int cus, bool loop) {
+// Waves of a decode workgroup and workgroups of a launch.
+struct DecodeShape {
+    int waves;
+    int64_t grid;
+};
+
+// The bf16 decode: workgroups that stay and loop over the tiles, one a CU, or
+// two where the LDS holds two whose waves take the tiles in fewer rounds (a
+// second table, but more waves to hide each other's latencies: 20480x2560 in
+// 20x512 tiles 29.9 us in one of 10 waves, twice over, 26.8 in two of 10;
+// 4096x4096 in 2x1024 tiles of two states 13.9 and 12.2).  Stored past the
+// caches (pair) only one: HBM takes the fewer writers' stores faster
+// (28672x4096 53.1 us in one, 57.6 in two).  No more waves than give each the
+// same number of tiles, but 4 to copy the table (64x256 4.6 us with one wave a
+// workgroup, 4.0 with four).
+DecodeShape decode_shape_loop(const rans_w64_matrix* m, int64_t ntiles, int cus, bool pair) {
+    const WaveLayout L = wave_layout(m);
+    DecodeShape best = {0, 0};
+    int64_t best_rounds = 0;
+    for (int per_cu = 1; per_cu <= (pair ? 1 : 2); per_cu++) {
+        int most = 0;
+        while (most < kMaxDecodeWaves &&
+               per_cu * (lds_bytes(most + 1, L) + kDecodeStaticLds) <= (size_t)kLdsMax)
+            most++;
+        if (!most) break;
+        const int64_t groups = (int64_t)cus * per_cu;
+        const int64_t rounds = (ntiles + groups * most - 1) / (groups * most);
+        if (best.waves && rounds >= best_rounds) break;
+        const int waves = std::max((int)((ntiles + groups * rounds - 1) / (groups * rounds)),
+                                   std::min(4, most));
+        best = {waves, std::min(groups, (ntiles + waves - 1) / waves)};
+        best_rounds = rounds;
+    }
+    return best;
+}
+
+// The decode to int32 codes, whose time is its writes: of the counts that put
+// the fewest waves on the busiest CU when the workgroups spread evenly the
+// largest, from 4 up (workgroups of fewer waves fill the LDS with tables).
+DecodeShape decode_shape_once(const rans_w64_matrix* m, int64_t ntiles, int cus) {
     const WaveLayout L = wave_layout(m);
     int most = 0;
-    while (most < kMaxDecodeWaves && lds_bytes(most + 1, L) + kDecodeStaticLds <= (size_t)kLdsMax)
-        most++;
-    if (!most) return 0;
-    if (loop) {
-        const int64_t rounds = (ntiles + (int64_t)cus * most - 1) / ((int64_t)cus * most);
-        return (int)((ntiles + cus * rounds - 1) / (cus * rounds));
-    }
-    int best = 0;
+    while (most < 10 && lds_bytes(most + 1, L) + kDecodeStaticLds <= (size_t)kLdsMax) most++;
+    DecodeShape best = {0, 0};
     int64_t best_load = 0;
-    for (int w = std::min(4, most); w <= std::min(10, most); w++) {
+    for (int w = std::max(std::min(4, most), 1); w <= most; w++) {
         const int64_t grid = (ntiles + w - 1) / w;
         const int64_t load = (grid + cus - 1) / cus * w;
-        if (!best || load <= best_load) best = w, best_load = load;
+        if (!best.waves || load <= best_load) best = {w, grid}, best_load = load;
     }
     return best;
 }
@@ -297,13 +323,12 @@ int launch_decode_p(const DecodeArgs& a, int waves, size_t lds, int grid, hipStr
 }
 
 template <int R, int S, int MODE>
-int launch_decode_t(const DecodeArgs& a, int waves, size_t lds, int grid, hipStream_t stream) {
+int launch_decode_t(const DecodeArgs& a, bool pair, int waves, size_t lds, int grid,
+                    hipStream_t stream) {
     if constexpr (MODE == 1) {
         const bool loop = (int64_t)grid * waves < a.ntiles;
-        // paired rows in 4-byte stores (rows are a multiple of 128 bytes: cols
-        // is one of 64)
         if constexpr (R > 1) {
-            if ((uintptr_t)a.out % 4 == 0 && (int64_t)a.rows * a.cols >= kPairWeights)
+            if (pair)
                 return loop ? launch_decode_p<R, S, MODE, true, true>(a, waves, lds, grid, stream)
                             : launch_decode_p<R, S, MODE, true, false>(a, waves, lds, grid, stream);
         }
@@ -313,10 +338,10 @@ int launch_decode_t(const DecodeArgs& a, int waves, size_t lds, int grid, hipStr
 }
 
 template <int MODE>
-int dispatch_decode(const DecodeArgs& a, int R, int S, int waves, size_t lds, int grid,
+int dispatch_decode(const DecodeArgs& a, int R, int S, bool pair, int waves, size_t lds, int grid,
                     hipStream_t st) {
 #define VRAMC_DEC_CASE(RR, SS) \
-    if (R == RR && S == SS) return launch_decode_t<RR, SS, MODE>(a, waves, lds, grid, st);
+    if (R == RR && S == SS) return launch_decode_t<RR, SS, MODE>(a, pair, waves, lds, grid, st);
 #define VRAMC_DEC_R(RR) VRAMC_DEC_CASE(RR, 1) VRAMC_DEC_CASE(RR, 2) VRAMC_DEC_CASE(RR, 4)
     VRAMC_DEC_R(1) VRAMC_DEC_R(2) VRAMC_DEC_R(3) VRAMC_DEC_R(4) VRAMC_DEC_R(8) VRAMC_DEC_R(16)
     VRAMC_DEC_CASE(20, 1) VRAMC_DEC_CASE(35, 1)
@@ -333,7 +358,13 @@ int launch_decode_common(const rans_w64_matrix* m, void* out, hipStream_t stream
     const int64_t ntiles = (int64_t)(m->rows / m->R) * (m->cols / m->C);
     const int cus = device_cus();
     if (cus <= 0) return (int)hipErrorInvalidDevice;
-    const int waves = decode_waves(m, ntiles, cus, MODE == 1);
+    // paired rows in 4-byte stores (rows are a multiple of 128 bytes: cols is
+    // one of 64)
+    const bool pair = MODE == 1 && m->R > 1 && (uintptr_t)out % 4 == 0 &&
+                      (int64_t)m->rows * m->cols >= kPairWeights;
+    const DecodeShape shape = MODE == 1 ? decode_shape_loop(m, ntiles, cus, pair)
+                                        : decode_shape_once(m, ntiles, cus);
+    const int waves = shape.waves;
     if (!waves) return RANS_EGEOMETRY;
     DecodeArgs a;
     a.words = m->words;
@@ -354,9 +385,8 @@ int launch_decode_common(const rans_w64_matrix* m, void* out, hipStream_t stream
     a.W = waves;
     a.has_esc = !(m->flags & RANS_F_NO_ESCAPES);
     a.L = wave_layout(m);
-    const int64_t groups = (ntiles + waves - 1) / waves;
-    const int grid = (int)(MODE == 1 ? std::min<int64_t>(cus, groups) : groups);
-    return dispatch_decode<MODE>(a, m->R, m->S, waves, lds_bytes(waves, a.L), grid, stream);
+    return dispatch_decode<MODE>(a, m->R, m->S, pair, waves, lds_bytes(waves, a.L), (int)shape.grid,
+                                 stream);
 }
 
 }  // namespace
