@@ -14,7 +14,7 @@ namespace {
 
 // Waves of a decode workgroup (tiles are taken linearly, any count works).
 constexpr int kMaxDecodeWaves = 16;
-constexpr int64_t kPairWeights = 64 << 20;
+constexpr int64_t kPairWeights = 108 << 20;
 constexpr int kNonTemporal = 2;  // cache policy of a raw buffer store
 constexpr int kDecodeStaticLds = (int)sizeof(TabEntry<false>) * (int)kProbM;
 
@@ -51,21 +51,22 @@ __device__ __forceinline__ uint32_t quad_swap(uint32_t v) {
 // What bounds a large decode is its writes: storing into a window of 16 tile
 // rows, which stays in the caches, 25600x5120 takes 58 us instead of 100, and
 // writing the same bytes without decoding about 50.  So a bf16 output that
-// takes more than half of the 256 MB memory-side cache (kPairWeights) goes
-// out in
+// fills the 256 MB memory-side cache but for a sixth or less (kPairWeights)
+// goes out in
 //   - PAIR: one 4-byte store for two rows.  Lanes l and l^1 hold neighbouring
 //     columns, so they exchange halves and the even lane stores both columns
 //     of the first row, the odd lane both of the second: half the store
 //     instructions, for two more VALU instructions per pair;
 //   - non-temporal stores, which keep the caches for the coded input.
-// 25600x5120 100.2 -> 89.8 us, 5120x25600 113.2 -> 97.5, 34816x5120 104 -> 95.
-// (Pairs alone change nothing, and pairs of column steps or stores of 512
-// contiguous bytes over 4 of them ran slower.)  Smaller outputs are stored
-// plainly: non-temporal stores make those decodes up to 12% faster too, but a
-// matrix product that reads the output next then finds it in HBM instead of
-// the cache (decode and product with 32 rows of x at 5120x5120: 36.0 against
-// 30.9 us, 8960x1536 and 512 rows 35.5 against 32.6; at 13824x5120, 141 MB,
-// and 64 rows 74.2 against 79.4).
+// 25600x5120 84.2 -> 56.3 us, with 1% escapes 100.3 -> 86.4; 5120x25600 88.9
+// -> 61.9; 34816x5120 100.7 -> 75.0.  (Pairs alone change nothing, and pairs of
+// column steps or stores of 512 contiguous bytes over 4 of them ran slower.)
+// Smaller outputs are stored plainly: escapes, written over their tile's
+// values, then find them in the cache, as does a matrix product that reads the
+// output next.  Plain and non-temporal, us: 28672x4096 (224 MB) 70.8 and 53.1,
+// with 1% escapes 86.9 and 76.6; 20480x5120 (200 MB) 49.5 and 46.2, with
+// escapes 58.4 and 69.0, with a product of 32 rows 82.3 and 95.9; 16384x4096
+// (128 MB) 31.7 and 30.4, 35.5 and 45.3, 54.1 and 62.1.
 //
 // LOOP: workgroups stay, one or two a CU; each wave takes tiles first, first +
 // stride, ... and copies the next tile's block as soon as it has decoded the
