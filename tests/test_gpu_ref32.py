@@ -229,7 +229,9 @@ def test_reference_format_unaligned_words(rans, lib, golden, dev):
 
 
 @pytest.mark.parametrize("rows,cols,R,C", [(8, 32, 1, 32), (5, 544, 1, 544), (8, 352, 2, 352),
-                                           (20, 448, 4, 224), (48, 96, 16, 96)])
+                                           (20, 448, 4, 224), (48, 96, 16, 96),
+                                           # workgroups of two and three waves that decode
+                                           (601, 32, 1, 32), (1203, 32, 1, 32)])
 @pytest.mark.parametrize("shift", [0, 1])
 def test_reference_format_short_blocks(rans, oracle, lib, dev, rows, cols, R, C, shift):
     """Column steps that 16 symbols ahead do not divide, one to seventeen of
