@@ -31,18 +31,16 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <atomic>
 #include <cstdint>
-#include <mutex>
 
 #include "../../include/vramc_rans.h"
+#include "rans_device.h"
 
 namespace {
 
 constexpr uint32_t kRefM = 4096;
 constexpr uint32_t kRefL = 1u << 16;
 constexpr int kRefMaxWaves = 4;
-constexpr int kRefLdsMax = 160 * 1024;
 constexpr int kRefStaticLds = 8 * (int)kRefM;  // the 8-byte table image
 constexpr int kRefSlotMax = 64 * 1024;         // LDS words per wave at most
 constexpr int kRefBufWord3 = 0x00020000;       // buffer resource word 3 for raw loads
@@ -313,41 +311,12 @@ __global__ void __launch_bounds__(64 * kRefMaxWaves) ref32_kernel(Ref32Args a) {
     }
 }
 
-// Opt in to the dynamic LDS once per kernel.
-std::mutex g_ref_attr_mu;
-const void* g_ref_attr_done[16];
-int g_ref_attr_n = 0;
-
-hipError_t ref_ensure_lds(const void* fn, size_t bytes) {
-    if (bytes + kRefStaticLds <= 65536) return hipSuccess;
-    std::lock_guard<std::mutex> lk(g_ref_attr_mu);
-    for (int i = 0; i < g_ref_attr_n; i++)
-        if (g_ref_attr_done[i] == fn) return hipSuccess;
-    const hipError_t e =
-        hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, kRefLdsMax - kRefStaticLds);
-    if (e == hipSuccess && g_ref_attr_n < 16) g_ref_attr_done[g_ref_attr_n++] = fn;
-    return e;
-}
-
-// CUs of the current device, cached per device; 0 when the query fails.
-std::atomic<int> g_ref_cus[64];
-
-int ref_cus() {
-    int dev = 0, cus = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0) return 0;
-    if (dev < 64 && (cus = g_ref_cus[dev].load(std::memory_order_relaxed)) > 0) return cus;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return 0;
-    if (dev < 64) g_ref_cus[dev].store(cus, std::memory_order_relaxed);
-    return cus;
-}
-
 template <int R, bool DECODE>
 int ref32_launch(const Ref32Args& a, hipStream_t stream) {
     const int W = a.W;
     const void* fn = reinterpret_cast<const void*>(&ref32_kernel<R, DECODE>);
     const size_t dyn = (size_t)W * a.slot * 2;
-    if (const hipError_t e = ref_ensure_lds(fn, dyn); e != hipSuccess) return (int)e;
+    if (const hipError_t e = ensure_lds(fn, dyn, kRefStaticLds); e != hipSuccess) return (int)e;
     const int nwaves = (a.nlanes + 63) / 64;
     hipLaunchKernelGGL((ref32_kernel<R, DECODE>), dim3((nwaves + W - 1) / W),
                        dim3(64 * kRefMaxWaves), dyn, stream, a);
@@ -399,9 +368,9 @@ int ref32_entry(int R, const void* words, const void* offs, const void* table, c
     // the workgroup's four only help to copy it (64x256 in 8x256 tiles, 64
     // symbols a stream: 11.5 us without them, 9.8 with; 1536x8960 in 8x8960
     // tiles 105.8 and 103.5)
-    const int cus = ref_cus();
+    const int cus = device_cus();
     const int64_t per_cu = cus > 0 ? ((nlanes + 63) / 64 + cus - 1) / cus : kRefMaxWaves;
-    int W = (kRefLdsMax - kRefStaticLds) / (int)(slot * 2);
+    int W = (kLdsMax - kRefStaticLds) / (int)(slot * 2);
     W = (int)std::min<int64_t>(std::min(W, kRefMaxWaves), per_cu);
     a.W = std::max(W, 1);
     switch (R) {
