@@ -98,9 +98,10 @@ def compile_lib(arch="gfx950", out=LIB):
         objs = [os.path.join(work, os.path.basename(s) + ".o") for s in SOURCES]
         procs = [subprocess.Popen([*hipcc, "-c", "-o", o, s], stderr=err)
                  for o, s in zip(objs, SOURCES)]
-        codes = [p.wait() for p in procs]
-        if any(codes):
-            raise subprocess.CalledProcessError(max(codes), hipcc)
+        ended = [(p.wait(), p.args) for p in procs]
+        for code, cmd in ended:
+            if code:
+                raise subprocess.CalledProcessError(code, cmd)
         subprocess.check_call([*hipcc, "-shared", "-o", tmp, *objs], stderr=err)
     os.replace(tmp, out)
     return out
