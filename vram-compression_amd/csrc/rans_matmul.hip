@@ -13,7 +13,8 @@
 // Bound by the decode's instructions while x is short (5120x5120 at 17 rows
 // 24.5 us, 18 of them what decoding to memory takes) and from there on by the
 // reads of x, which every wave makes from the caches for its own columns, at
-// some 7 TB/s: hence T tile rows to a wave where those reads are many.
+// 7 to 9 TB/s: hence T tile rows to a wave where those reads cost more than
+// the waves given up for them.
 //
 // Shape: a workgroup holds one table copy and rpw groups of T whole tile rows,
 // a wave to each T tiles of a column, up to 16 waves; the waves of a tile row
