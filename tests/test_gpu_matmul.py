@@ -76,6 +76,21 @@ def test_refuses(rans, lib):
         m.matmul(torch.zeros(65, 1024, device="cuda"))
 
 
+def test_bias(rans, lib):
+    """A bias in another type or stride counts as its f32 values; one of
+    another length or on the host is refused before any launch."""
+    m = _matrix(rans, lib, 48, 1024, 16, 256, 0.0, 1)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randint(-4, 5, (20, 1024), device="cuda", generator=g).bfloat16()
+    b = torch.randint(-8, 9, (48, 2), device="cuda", generator=g).float()
+    want = m.matmul(x) + b[:, 0]
+    for bias in (b[:, 0], b[:, 0].bfloat16(), b[:, 0].contiguous().half(), b[:, 0].double()):
+        assert torch.equal(m.matmul(x, bias), want)
+    for bias in (b[:47, 0], b[:1, 0], b[:, 0].cpu(), b[:, :1], torch.zeros(64, device="cuda")):
+        with pytest.raises(ValueError):
+            m.matmul(x, bias)
+
+
 def test_linear_route(rans, lib):
     """Misaligned rows, f16 and f32 inputs and leading dimensions on the fused
     product; a watched x on the dense one, with its gradient."""
