@@ -60,11 +60,13 @@ def test_finish_takes_the_products_it_has_a_kernel_for(on_cpu, y_dtype, bias):
         got = on_cpu._finish(lib, y, b, out)
         assert got.dtype is out and got.shape == y.shape
         if y_dtype in (torch.float32, torch.bfloat16):
-            assert bool(lib.calls) == (bias or y_dtype is not out)
+            assert bool(lib.calls) == (y_dtype is not out or bias and out is not torch.float32)
         else:
             assert not lib.calls
             assert torch.equal(got, (y.float() if b is None else y.float() + b).to(out))
         lib.calls.clear()
+        if bias:
+            assert on_cpu._finish(lib, y, b.double(), out).dtype is out and not lib.calls
 
 
 class _Matrix:
